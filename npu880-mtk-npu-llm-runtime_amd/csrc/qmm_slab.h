@@ -1,0 +1,75 @@
+// qmm_slab.h — what the prefill kernels share (qmm_slab.hip, qmm_wslab.hip):
+// a row tile's block unpacked from LDS into MFMA operand registers.
+#pragma once
+
+#include "qmm_kformats.h"
+
+namespace qmm {
+
+typedef _Float16 half4v __attribute__((ext_vector_type(4)));
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+
+// B operands of one row tile for one block
+struct SlabB {
+    uint4 b1[4], b2[4];
+    half4v mh;  // mins of the lane's groups (Q4_K / Q5_K)
+    float d, dmin;
+};
+
+// the 4 mins (as fp16) a lane supplies for groups 4c .. 4c + 3: units 2c, 2c,
+// 2c + 1, 2c + 1 (mw: the 8 mins four to a dword)
+__device__ inline half4v mins_f16(const uint32_t (&mw)[2], int c) {
+    // (a mask select: an index would put mw in scratch memory)
+    const uint32_t sel = 0u - uint32_t((c >> 1) & 1);
+    const uint32_t w = (mw[0] & ~sel) | (mw[1] & sel);
+    const int b0 = 2 * (c & 1);
+    const half2v bias = {(_Float16)1024.0f, (_Float16)1024.0f};
+    // 0x6400 | m is the fp16 value 1024 + m (m < 64): subtract 1024, exactly
+    const half2v lo = __builtin_bit_cast(half2v, __builtin_bit_cast(uint32_t, byte_pair(w, b0)) | 0x64006400u) - bias;
+    const half2v hi =
+        __builtin_bit_cast(half2v, __builtin_bit_cast(uint32_t, byte_pair(w, b0 + 1)) | 0x64006400u) - bias;
+    return half4v{lo.x, lo.y, hi.x, hi.y};
+}
+
+template <class F>
+__device__ inline void slab_unpack(const uint8_t *blk, int c, SlabB &o) {
+    if constexpr (std::is_same_v<F, MQ6KS>) {
+        const MQ6KS::W w = MQ6KS::load_lds(blk, c);
+        SplitB sb;
+        split_b(w, c, sb);
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            o.b1[h] = sb.b1[h];
+            o.b2[h] = sb.b2[h];
+        }
+        o.d = fp16_bits_to_f32(w.d);
+        o.dmin = 0.0f;
+    } else {  // Q4_K / Q5_K folded
+        const typename F::W w = F::load_lds(blk, c);
+        uint32_t scp[2], mp[2];
+        scales_k4_packed(w.h.y, w.h.z, w.h.w, scp, mp);
+        SplitB sb;
+        split_b(w, scp, mp, sb);
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            o.b1[h] = sb.b1[h];
+            o.b2[h] = sb.b2[h];
+        }
+        o.mh = mins_f16(mp, c);
+        o.d = fp16_bits_to_f32(w.h.x & 0xFFFFu);
+        o.dmin = fp16_bits_to_f32(w.h.x >> 16);
+    }
+}
+
+// the wave-slab shape of a call and its expected time per 256-value block
+struct WslabPlan {
+    char shape;
+    int64_t ns;
+};
+template <class F>
+WslabPlan wslab_plan(const MatArgs *tasks, int n);
+template <class F>
+hipError_t launch_wslab(const WslabPlan &p, const MatArgs *tasks, int n, const Q8KView &x, hipStream_t s);
+
+}  // namespace qmm

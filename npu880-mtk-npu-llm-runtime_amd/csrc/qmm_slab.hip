@@ -27,13 +27,9 @@
 // Workgroups are numbered so that the ones sharing a row slab run together on
 // one XCD (workgroup b runs on XCD b mod 8): that XCD's L2 then serves the
 // slab's weights to every token group after the first read from HBM.
-#include "qmm_kformats.h"
+#include "qmm_slab.h"
 
 namespace qmm {
-
-typedef _Float16 half4v __attribute__((ext_vector_type(4)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef float f32x4v __attribute__((ext_vector_type(4)));
 
 template <class F, int RW_, int TW_, int PR_, int PD_, int NW_ = 4, int WPS_ = 1>
 struct SlabCfg {
@@ -66,58 +62,6 @@ struct SlabCfg {
     static_assert((PD - 2) * L <= 63, "vmcnt range");
     static_assert(LDS <= 160 * 1024, "LDS");
 };
-
-// B operands of one row tile for one block
-struct SlabB {
-    uint4 b1[4], b2[4];
-    half4v mh;  // mins of the lane's groups (Q4_K / Q5_K)
-    float d, dmin;
-};
-
-// the 4 mins (as fp16) a lane supplies for groups 4c .. 4c + 3: units 2c, 2c,
-// 2c + 1, 2c + 1 (mw: the 8 mins four to a dword)
-__device__ inline half4v mins_f16(const uint32_t (&mw)[2], int c) {
-    // (a mask select: an index would put mw in scratch memory)
-    const uint32_t sel = 0u - uint32_t((c >> 1) & 1);
-    const uint32_t w = (mw[0] & ~sel) | (mw[1] & sel);
-    const int b0 = 2 * (c & 1);
-    const half2v bias = {(_Float16)1024.0f, (_Float16)1024.0f};
-    // 0x6400 | m is the fp16 value 1024 + m (m < 64): subtract 1024, exactly
-    const half2v lo = __builtin_bit_cast(half2v, __builtin_bit_cast(uint32_t, byte_pair(w, b0)) | 0x64006400u) - bias;
-    const half2v hi =
-        __builtin_bit_cast(half2v, __builtin_bit_cast(uint32_t, byte_pair(w, b0 + 1)) | 0x64006400u) - bias;
-    return half4v{lo.x, lo.y, hi.x, hi.y};
-}
-
-template <class F>
-__device__ inline void slab_unpack(const uint8_t *blk, int c, SlabB &o) {
-    if constexpr (std::is_same_v<F, MQ6KS>) {
-        const MQ6KS::W w = MQ6KS::load_lds(blk, c);
-        SplitB sb;
-        split_b(w, c, sb);
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-            o.b1[h] = sb.b1[h];
-            o.b2[h] = sb.b2[h];
-        }
-        o.d = fp16_bits_to_f32(w.d);
-        o.dmin = 0.0f;
-    } else {  // Q4_K / Q5_K folded
-        const typename F::W w = F::load_lds(blk, c);
-        uint32_t scp[2], mp[2];
-        scales_k4_packed(w.h.y, w.h.z, w.h.w, scp, mp);
-        SplitB sb;
-        split_b(w, scp, mp, sb);
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-            o.b1[h] = sb.b1[h];
-            o.b2[h] = sb.b2[h];
-        }
-        o.mh = mins_f16(mp, c);
-        o.d = fp16_bits_to_f32(w.h.x & 0xFFFFu);
-        o.dmin = fp16_bits_to_f32(w.h.x >> 16);
-    }
-}
 
 template <class C, class F>
 __global__ __launch_bounds__(64 * C::NW, C::WPS) void slab_kernel(MatGroup grp, typename ActOf<F>::T x, int ntg) {
@@ -860,7 +804,6 @@ static hipError_t launch_slab_t(const MatArgs *tasks, int n, const typename ActO
 }
 
 int mfma_cu_count();
-
 // hipErrorNotSupported (nothing launched) where the slab kernels do not
 // apply: K not a multiple of 256, operand sections missing, rows of an
 // aligned format not 16-B aligned, offsets past the 32-bit buffer range, 64
@@ -877,14 +820,6 @@ hipError_t launch_slab(const MatArgs *tasks, int n, const typename ActOf<F>::T &
         if (aligned && ((reinterpret_cast<uintptr_t>(tasks[i].w) | tasks[i].row_bytes) & 15)) return hipErrorNotSupported;
         if (size_t(tasks[i].N) * tasks[i].row_bytes + 16 >= (size_t(1) << 31)) return hipErrorNotSupported;
     }
-    // Packed slabs (the shape is chosen at the end): 128 rows x 64 tokens in
-    // 8 waves, two per CU (2 x 74 KB of LDS, <= 128 VGPRs), so four waves per
-    // SIMD and the 64 tokens' codes staged once per 128 rows (gate + up 2 x
-    // 9728 x 2560 at M = 512: 87.5 -> 79.1 us); 64 x 64 (two per CU); 64 x 32
-    // (three or four per CU: O 2560 x 4096 at M = 512: 28.5 -> 23.9 us).
-    // Measured slower at M = 512: 128 x 128 in 8 waves, 128 x 32 in 8 waves,
-    // 32 x 128, 32 x 64, 64 x 16, 32 x 32, three stages, and two row tiles
-    // per wave.
     // Q6_K at 33..64 tokens: decoded slabs of 16 rows x 64 tokens in 16
     // waves, four K groups of four, steps two deep (down 2560 x 9728 at M =
     // 48 / 64: 20.1 / 20.8 us; one deep 21.9 / 22.2; 23 / 27.1 for the 16 x 16
@@ -914,47 +849,45 @@ hipError_t launch_slab(const MatArgs *tasks, int n, const typename ActOf<F>::T &
         }
         return hipErrorNotSupported;
     }
-    // Q6_K / Q5_K from 128 tokens: decoded slabs (their decoding is costly
-    // next to the epilogue). Measured at M = 128 / 200 / 300 / 512 / 1024:
-    // down 2560 x 9728 (16 rows x 128 tokens) 34.4 / 42.6 / 43.5 / 58.4 /
-    // 103.8 us against 39.0 / 56.6 / 57.5 / 77.8 / 126.3 (slab kernel); QKV
-    // 6144 x 2560 (32 x 128) 16.8 / 22.5 / 33.1 / 33.9 / 59.0 against 18.7 /
-    // 24.0 / 31.2 / 37.2 / 63.1. Q4_K stays on the slab kernel (gate + up and
-    // O at M = 512: 86.5 and 29.0 us against 78.9 and 28.0): its epilogue
-    // outweighs its decoding, and the slab kernel fits more waves per SIMD.
-    // Q6_K from 65 tokens (the tokens padded to 128): faster than the packed
-    // slabs at every height measured (down 2560 x 9728 at M = 65..127 38.6 ->
-    // 33.1 us; 1024 x 9728 38.6 -> 32.7, 1024 x 2560 12.9 -> 11.6, 4096 x
-    // 2560 13.0 -> 11.9 at M = 65..512). Q5_K where its workgroups number at
-    // least 5/8 of the CUs (QKV 6144 x 2560 at M = 65..127 17.4 -> 16.1 us;
-    // 4096 x 2560 at M = 128 12.8 against 16.2, 1024 x 2560 12.3 against 15.8
-    // on the packed slabs: there they stay).
-    if constexpr (std::is_same_v<F, MQ6KS> || std::is_same_v<F, MQ5KS>) {
-        int wgs = 0;
-        for (int i = 0; i < n; ++i) wgs += (tasks[i].N + 31) / 32;
-        if (std::is_same_v<F, MQ6KS> || 8 * wgs * ((a.M + 127) / 128) >= 5 * mfma_cu_count()) {
-            hipError_t e = hipErrorNotSupported;
-            if constexpr (std::is_same_v<F, MQ6KS>) e = launch_dslab_t<DsCfg<F, 1, 4, 2>, F>(tasks, n, x, s);
-            if constexpr (std::is_same_v<F, MQ5KS>) e = launch_dslab_t<DsCfg<F, 2, 4, 2>, F>(tasks, n, x, s);
-            if (e != hipErrorNotSupported) return e;
-        }
-    }
-    int slabs = 0, slabs128 = 0;
+    // Past 64 tokens: the wave slabs (qmm_wslab.hip) where their expected time
+    // per block is at least 8 % below that of this file's kernels, which win
+    // where the workgroups are few (their steps are shorter, their tiles
+    // smaller). Their times per block, fitted over the same sweep with w
+    // workgroups per CU and a call's fixed 4 us taken off: decoded slabs Q6_K
+    // 16 x 128 0.1 + 0.56 w us (2560 x 9728 at M = 512 / 1024 / 2048: 1.34 /
+    // 2.55 / 5.95), Q5_K 32 x 128 0.3 + 0.92 w (6144 x 2560 at M = 200 / 512 /
+    // 2048: 1.7 / 2.9 / 11.5, 3001 x 8192 at M = 777 2.6), packed 64 x 32
+    // slabs 0.35 + 0.5 w (Q4_K 2560 x 4096 at M = 512 / 1024: 1.3 / 2.5, 2 x
+    // 9728 x 2560 at M = 65: 1.9).
+    // Q6_K and Q5_K decode in LDS (their decoding is costly next to their
+    // update) from 65 tokens, Q5_K where those workgroups number at least 5/8
+    // of the CUs (QKV 6144 x 2560 at M = 65..127 17.4 -> 16.1 us; 4096 x 2560
+    // at M = 128 12.8 against 16.2, 1024 x 2560 12.3 against 15.8 on the
+    // packed slabs: there they stay). Q4_K stays packed: its update outweighs
+    // its decoding (2560 x 4096 at M = 512 25.1 against 26.9 us and more).
+    const int cus = mfma_cu_count();
+    int w16 = 0, w32 = 0, w64 = 0;
     for (int i = 0; i < n; ++i) {
-        slabs += (tasks[i].N + 63) / 64;
-        slabs128 += (tasks[i].N + 127) / 128;
+        w16 += (tasks[i].N + 15) / 16;
+        w32 += (tasks[i].N + 31) / 32;
+        w64 += (tasks[i].N + 63) / 64;
     }
-    const int tg64 = (a.M + 63) / 64, cus = mfma_cu_count();
-    const int w128 = slabs128 * tg64, w64 = slabs * tg64;  // workgroups of the 128 x 64 / 64 x 64 shapes
-    // 128 x 64 in 8 waves where those workgroups number at least 1.5 per CU;
-    // 64 x 64 where they make one round of two per CU (1.75..2 per CU); else
-    // 64 x 32. Measured (Q4_K, M = 65..512, K = 2560, kernel alone): 19456
-    // rows at M = 65 / 128 / 384 32.5 / 33.5 / 72.5 -> 23.0 / 30.0 / 59.8 us,
-    // 9728 rows at M = 256 33.2 -> 28.0, 6144 rows at M = 384 32.2 -> 27.0;
-    // M = 512 of gate + up and O unchanged (128 x 64 and 64 x 32).
-    //                                                         RW TW PR PD NW WPS
-    if (2 * w128 >= 3 * cus) return launch_slab_t<SlabCfg<F, 1, 4, 8, 2, 8, 4>, F>(tasks, n, x, s);
-    if (4 * w64 >= 7 * cus && w64 <= 2 * cus) return launch_slab_t<SlabCfg<F, 1, 4, 4, 2>, F>(tasks, n, x, s);
+    const int t128 = (a.M + 127) / 128, t32 = (a.M + 31) / 32;
+    const bool decoded = std::is_same_v<F, MQ6KS> || (std::is_same_v<F, MQ5KS> && 8 * w32 * t128 >= 5 * cus);
+    const int64_t ns = std::is_same_v<F, MQ6KS> ? 100 + int64_t(560) * w16 * t128 / cus
+                       : decoded                ? 300 + int64_t(920) * w32 * t128 / cus
+                                                : 350 + int64_t(500) * w64 * t32 / cus;
+    const WslabPlan plan = wslab_plan<F>(tasks, n);
+    if (108 * plan.ns < 100 * ns) return launch_wslab<F>(plan, tasks, n, x, s);
+    if (decoded) {
+        hipError_t e = hipErrorNotSupported;
+        if constexpr (std::is_same_v<F, MQ6KS>) e = launch_dslab_t<DsCfg<F, 1, 4, 2>, F>(tasks, n, x, s);
+        if constexpr (std::is_same_v<F, MQ5KS>) e = launch_dslab_t<DsCfg<F, 2, 4, 2>, F>(tasks, n, x, s);
+        if (e != hipErrorNotSupported) return e;  // (its scales past the LDS: the packed slabs)
+    }
+    // 64 rows x 32 tokens in 4 waves, three or four workgroups per CU (O 2560
+    // x 4096 at M = 512: 28.5 -> 23.9 us against 64 x 64). Measured slower at
+    // M = 512: 32 x 64, 64 x 16, 32 x 32, three stages, two row tiles per wave.
     return launch_slab_t<SlabCfg<F, 1, 2, 4, 2>, F>(tasks, n, x, s);
 }
 

@@ -1,0 +1,53 @@
+"""The wave-slab prefill GEMM (csrc/qmm_wslab.hip) vs the oracle, bit for bit:
+its three shapes (128 rows x 96 tokens, 128 x 64, 64 x 64) on every k-quant
+format, with rows and tokens past the last tile, one block and several, a
+task group, a residual, and Q6_K rows off every 16-B boundary."""
+import numpy as np
+import pytest
+
+import qmm_hip
+import synth
+from gpu_util import check_outputs, say
+from oracle import TYPE_Q4_K, TYPE_Q5_K, TYPE_Q6_K
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(ctx, oracle, type_id, rows, K, M, residual, skip=0):
+    say(f"type {type_id} rows={rows} K={K} M={M} residual={residual} from row {skip}")
+    x = synth.activations(M, K, seed=K + M)
+    xb = ctx.upload(x)
+    rb = qmm_hip.row_bytes(type_id, K)
+    bufs, tasks, ref = [xb], [], []
+    for i, N in enumerate(rows):
+        w = synth.weights(type_id, N + skip, K, seed=31 * i + N)
+        wb, yb = ctx.weight_upload(w, type_id, N + skip, K), ctx.malloc(M * N * 4)
+        res = synth.activations(M, N, seed=7 * i + N) if residual else None
+        resb = ctx.upload(res) if residual else None
+        bufs += [b for b in (wb, yb, resb) if b is not None]
+        tasks.append(qmm_hip.MatrixTask(wb.ptr + skip * rb, type_id, N, K, yb, N, resb, N if residual else 0))
+        ref.append(dict(w=w[skip * rb:], type=type_id, rows=N, **(dict(residual=res) if residual else {})))
+    ctx.gemm_multi_dispatch(xb, M, K, tasks)
+    ctx.sync()
+    for t, r in zip(tasks, oracle.gemm_multi(x, ref)):
+        check_outputs(ctx.d2h(t.dst, np.float32, (M, t.rows)), r, f"rows={t.rows} K={K} M={M}")
+    for b in bufs:
+        ctx.free(b)
+
+
+@pytest.mark.parametrize("type_id,rows,K,M,residual", [
+    # 128 rows x 96 tokens: ragged last tokens (80, 40, 70 of 96) and rows
+    (TYPE_Q4_K, [3000], 512, 2000, True), (TYPE_Q6_K, [5001], 768, 1000, False), (TYPE_Q5_K, [4100], 256, 1030, True),
+    # 128 x 64
+    (TYPE_Q4_K, [5003], 768, 700, False), (TYPE_Q6_K, [6001], 512, 600, True), (TYPE_Q5_K, [6100], 256, 2000, False),
+    # 64 x 64: one token past a group, a 49-row task in the group
+    (TYPE_Q4_K, [8190], 256, 257, True), (TYPE_Q5_K, [8201], 512, 300, False), (TYPE_Q6_K, [9001], 768, 300, False),
+    (TYPE_Q4_K, [2500, 49], 512, 1000, True)])
+def test_wave_slabs(ctx, oracle, type_id, rows, K, M, residual):
+    _run(ctx, oracle, type_id, rows, K, M, residual)
+
+
+@pytest.mark.parametrize("rows,K,M", [([5000], 768, 1000), ([6000], 256, 600), ([9000], 768, 300)])
+def test_wave_slabs_unaligned_q6k(ctx, oracle, rows, K, M):
+    """Q6_K rows from row 1 of a tensor: 210-B blocks 2 B off a 4-B boundary."""
+    _run(ctx, oracle, TYPE_Q6_K, rows, K, M, False, skip=1)
