@@ -340,6 +340,28 @@ __device__ inline int group8_sum(int v) {
     return v;
 }
 
+// op over all 64 lanes, in every lane: the butterfly over lane distances 32,
+// 16, 8, 4, 2, 1 (op commutative: each lane's result is the same tree), in
+// registers — permlane swaps, row rotations (after the step over 8 a row
+// repeats every 8 lanes, so a rotation by 4 is the exchange over 4) and quad
+// permutes — instead of six dependent LDS permutes.
+template <class Op>
+__device__ inline float wave_all(float v, Op op) {
+    auto f = [](uint32_t b) { return __builtin_bit_cast(float, b); };
+    auto dpp = [&](auto ctrl, float a) {
+        return f(uint32_t(__builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, a), decltype(ctrl)::value, 0xF, 0xF, false)));
+    };
+    const uint32_t a = __builtin_bit_cast(uint32_t, v);
+    const auto r32 = __builtin_amdgcn_permlane32_swap(a, a, false, false);
+    const uint32_t b = __builtin_bit_cast(uint32_t, op(f(r32[0]), f(r32[1])));
+    const auto r16 = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    v = op(f(r16[0]), f(r16[1]));
+    v = op(v, dpp(std::integral_constant<int, 0x128>{}, v));  // row_ror:8
+    v = op(v, dpp(std::integral_constant<int, 0x124>{}, v));  // row_ror:4
+    v = op(v, dpp(std::integral_constant<int, 0x4E>{}, v));   // quad_perm 2, 3, 0, 1
+    return op(v, dpp(std::integral_constant<int, 0xB1>{}, v));  // quad_perm 1, 0, 3, 2
+}
+
 // --------------------------------------------------------- global loads
 typedef uint32_t v4u32 __attribute__((ext_vector_type(4)));
 // 16 B load of an address that is 16-B aligned.
@@ -377,8 +399,7 @@ __device__ inline float rms_add4(float s, float4 h) {
     return s;
 }
 __device__ inline float rms_inv(float s, int K, float *part) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
+    s = wave_all(s, [](float a, float b) { return a + b; });
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
     lds_barrier();
     const float sum_sq = (part[0] + part[1]) + (part[2] + part[3]);
@@ -565,15 +586,13 @@ __device__ inline uint32_t quant4(float h0, float h1, float h2, float h3, float 
 __device__ inline float q8_scale(float amax) { return amax == 0.0f ? 0.0f : amax / 127.0f; }
 
 __device__ inline float wave_max(float a) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) a = fmaxf(a, __shfl_xor(a, off));
-    return a;
+    return wave_all(a, [](float x, float y) { return fmaxf(x, y); });
 }
 __device__ inline float group8_max(float a) {
-    a = fmaxf(a, __shfl_xor(a, 1));
-    a = fmaxf(a, __shfl_xor(a, 2));
-    a = fmaxf(a, __shfl_xor(a, 4));
-    return a;
+    auto f = [](int b) { return __builtin_bit_cast(float, b); };
+    a = fmaxf(a, f(dpp_xor1(__builtin_bit_cast(int, a))));
+    a = fmaxf(a, f(dpp_xor2(__builtin_bit_cast(int, a))));
+    return fmaxf(a, f(dpp_half_mirror(__builtin_bit_cast(int, a))));
 }
 
 // get_scale_min_k4 (E:743-749) for sub-block j given the 12 scale bytes
