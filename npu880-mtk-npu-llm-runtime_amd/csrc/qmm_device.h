@@ -442,14 +442,24 @@ __device__ inline Best better(Best a, Best b) {
     if (a.i == kNone || b.v > a.v || (b.v == a.v && b.i < a.i)) return b;
     return a;
 }
+// (better is commutative: wave_all's butterfly, on both words)
 __device__ inline Best wave_best(Best b) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        Best o;
-        o.v = __shfl_xor(b.v, off, 64);
-        o.i = uint32_t(__shfl_xor(int(b.i), off, 64));
-        b = better(b, o);
-    }
+    auto f = [](uint32_t u) { return __builtin_bit_cast(float, u); };
+    auto u = [](float v) { return __builtin_bit_cast(uint32_t, v); };
+    auto dpp = [&](auto ctrl, uint32_t a) {
+        return uint32_t(__builtin_amdgcn_mov_dpp(int(a), decltype(ctrl)::value, 0xF, 0xF, false));
+    };
+    const auto v32 = __builtin_amdgcn_permlane32_swap(u(b.v), u(b.v), false, false);
+    const auto i32 = __builtin_amdgcn_permlane32_swap(b.i, b.i, false, false);
+    b = better(Best{f(v32[0]), i32[0]}, Best{f(v32[1]), i32[1]});
+    const auto v16 = __builtin_amdgcn_permlane16_swap(u(b.v), u(b.v), false, false);
+    const auto i16 = __builtin_amdgcn_permlane16_swap(b.i, b.i, false, false);
+    b = better(Best{f(v16[0]), i16[0]}, Best{f(v16[1]), i16[1]});
+    auto step = [&](auto ctrl) { b = better(b, Best{f(dpp(ctrl, u(b.v))), dpp(ctrl, b.i)}); };
+    step(std::integral_constant<int, 0x128>{});  // row_ror:8
+    step(std::integral_constant<int, 0x124>{});  // row_ror:4
+    step(std::integral_constant<int, 0x4E>{});   // quad_perm 2, 3, 0, 1
+    step(std::integral_constant<int, 0xB1>{});   // quad_perm 1, 0, 3, 2
     return b;
 }
 

@@ -36,8 +36,14 @@ __global__ __launch_bounds__(256) void argmax_partial_kernel(float *__restrict__
     float *lr = logits + size_t(m) * ldl;
     const int r0 = s * kSlice, r1 = min(rows, r0 + kSlice);
     Best b{-INFINITY, kNone};
-    for (int r = r0 + int(threadIdx.x); r < r1; r += 256) {  // increasing r: ties keep the first
-        float v = lr[r];
+    float lv[kSlice / 256];  // every load before the first comparison
+#pragma unroll
+    for (int k = 0; k < kSlice / 256; ++k) lv[k] = lr[min(r0 + int(threadIdx.x) + 256 * k, r1 - 1)];
+#pragma unroll
+    for (int k = 0; k < kSlice / 256; ++k) {  // increasing r: ties keep the first
+        const int r = r0 + int(threadIdx.x) + 256 * k;
+        if (r >= r1) break;
+        float v = lv[k];
         if (ids && ids[r] >= id_limit) {
             v = -1e30f;
             lr[r] = v;
