@@ -21,7 +21,7 @@
 // broadcast 6-bit mins (exact; equal to the reference's bsum form for every
 // Q8_K row whose block sums are the sums of its codes, which the quantizer
 // guarantees).
-#include "qmm_kformats.h"
+#include "qmm_slab.h"
 
 namespace qmm {
 
@@ -1045,7 +1045,8 @@ static hipError_t launch_tile_t(const MatArgs *tasks, int n, const typename ActO
     return hipGetLastError();
 }
 
-// the prefill kernel (qmm_slab.hip); hipErrorNotSupported where it does not apply
+// wave slabs up to 64 tokens on tall tensors (qmm_wslab.hip), the prefill
+// kernel (qmm_slab.hip); hipErrorNotSupported where it does not apply
 template <class F>
 hipError_t launch_slab(const MatArgs *tasks, int n, const typename ActOf<F>::T &x, hipStream_t s);
 
@@ -1053,6 +1054,8 @@ template <class F>
 static hipError_t launch_tile(const MatArgs *tasks, int n, const typename ActOf<F>::T &x, hipStream_t s) {
     const MatArgs &a = tasks[0];
     if constexpr (std::is_same_v<F, MQ4K> || std::is_same_v<F, MQ5K> || std::is_same_v<F, MQ6KS>) {
+        const hipError_t tall = launch_wslab_tall<typename Folded<F>::T>(tasks, n, x, s);
+        if (tall != hipErrorNotSupported) return tall;
         // (Q6_K at 17..64 tokens over K > 4096, Q4_K / Q5_K at 33..64 over
         // K >= 8192: the decoded slabs split over K, where the launcher
         // takes them; Q6_K over K <= 4096 measured faster on the part kernel:

@@ -62,6 +62,26 @@ __device__ inline void slab_unpack(const uint8_t *blk, int c, SlabB &o) {
     }
 }
 
+// whether the slab kernels apply: K a multiple of 256, the operand sections
+// present, rows of an aligned format 16-B aligned, offsets inside the 32-bit
+// buffer range
+template <class F>
+inline bool slab_ok(const MatArgs *tasks, int n, const Q8KView &x) {
+    const MatArgs &a = tasks[0];
+    if (a.K % 256 || !x.qt || (F::kMin && !x.bh)) return false;
+    if (size_t((a.M + 15) & ~15) * size_t(a.K) >= (size_t(1) << 31)) return false;
+    for (int i = 0; i < n; ++i) {
+        if (F::BB % 16 == 0 && ((reinterpret_cast<uintptr_t>(tasks[i].w) | tasks[i].row_bytes) & 15)) return false;
+        if (size_t(tasks[i].N) * tasks[i].row_bytes + 16 >= (size_t(1) << 31)) return false;
+    }
+    return true;
+}
+
+// up to 64 tokens on tall tensors; hipErrorNotSupported (nothing launched)
+// where the small-M kernels are to run
+template <class F>
+hipError_t launch_wslab_tall(const MatArgs *tasks, int n, const Q8KView &x, hipStream_t s);
+
 // the wave-slab shape of a call and its expected time per 256-value block
 struct WslabPlan {
     char shape;

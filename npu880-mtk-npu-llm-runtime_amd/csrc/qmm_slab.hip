@@ -805,21 +805,12 @@ static hipError_t launch_slab_t(const MatArgs *tasks, int n, const typename ActO
 
 int mfma_cu_count();
 // hipErrorNotSupported (nothing launched) where the slab kernels do not
-// apply: K not a multiple of 256, operand sections missing, rows of an
-// aligned format not 16-B aligned, offsets past the 32-bit buffer range, 64
-// tokens or fewer other than Q6_K, or a decoded slab's LDS over the CU's.
+// apply (slab_ok), at 64 tokens or fewer outside the shapes below, or with a
+// decoded slab's LDS over the CU's.
 template <class F>
 hipError_t launch_slab(const MatArgs *tasks, int n, const typename ActOf<F>::T &x, hipStream_t s) {
     const MatArgs &a = tasks[0];
-    if (a.K % 256 || !x.qt) return hipErrorNotSupported;
-    if constexpr (F::kMin)
-        if (!x.bh) return hipErrorNotSupported;
-    if (size_t((a.M + 15) & ~15) * size_t(a.K) >= (size_t(1) << 31)) return hipErrorNotSupported;
-    constexpr bool aligned = F::BB % 16 == 0;
-    for (int i = 0; i < n; ++i) {
-        if (aligned && ((reinterpret_cast<uintptr_t>(tasks[i].w) | tasks[i].row_bytes) & 15)) return hipErrorNotSupported;
-        if (size_t(tasks[i].N) * tasks[i].row_bytes + 16 >= (size_t(1) << 31)) return hipErrorNotSupported;
-    }
+    if (!slab_ok<F>(tasks, n, x)) return hipErrorNotSupported;
     // Q6_K at 33..64 tokens: decoded slabs of 16 rows x 64 tokens in 16
     // waves, four K groups of four, steps two deep (down 2560 x 9728 at M =
     // 48 / 64: 20.1 / 20.8 us; one deep 21.9 / 22.2; 23 / 27.1 for the 16 x 16

@@ -29,10 +29,11 @@
 
 namespace qmm {
 
-// TT token tiles, NW waves, WPS waves per SIMD that the registers must allow
-template <class F, int TT_, int NW_, int WPS_>
+// TT token tiles, NW waves, WPS waves per SIMD that the registers must allow,
+// PD stages of the tokens' operands (and PD - 1 of the rows)
+template <class F, int TT_, int NW_, int WPS_, int PD_ = 2>
 struct WsCfg {
-    static constexpr int TT = TT_, NW = NW_, WPS = WPS_;
+    static constexpr int TT = TT_, NW = NW_, WPS = WPS_, PD = PD_;
     static constexpr int R = 16 * NW, T = 16 * TT;
     static constexpr bool MIN = F::kMin;
     static constexpr int SB = F::BB;
@@ -44,9 +45,12 @@ struct WsCfg {
     static constexpr int NBI = MIN ? (TT + 1) / 2 : 0;      // transfers of the sums of 16 codes
     static constexpr int NDI = (T + 63) / 64;     // transfers of the block scales (256 B)
     static constexpr int OFF_B = NAI * 1024, OFF_D = OFF_B + NBI * 1024, STAGE = OFF_D + NDI * 256;
-    static constexpr int OFF_W = 2 * STAGE, WREG = WSU * 16;
-    static constexpr int LDS = OFF_W + NW * WREG;
+    static constexpr int OFF_W = PD * STAGE, WREG = WSU * 16;
+    static constexpr int LDS = OFF_W + (PD - 1) * NW * WREG;
+    // transfers that every wave issues per block at least (some issue more)
+    static constexpr int L = NWW + NAI / NW + (NBI + NDI) / NW;
     static_assert(LDS <= 160 * 1024, "LDS");
+    static_assert(PD >= 2 && (PD - 2) * L <= 63, "vmcnt range");
 };
 
 template <class C, class F>
@@ -83,8 +87,10 @@ __global__ __launch_bounds__(64 * C::NW, C::WPS) void wslab_kernel(MatGroup grp,
     const v4i32 rd = buf_rsrc(x.d, uint32_t(a.M) * uint32_t(nbk) * 4u);
     const uint32_t lds0 = lds_addr(lds);
 
-    // the wave's packed rows of block j into its region
-    const uint32_t wbase = uint32_t(C::OFF_W + wid * C::WREG);
+    // the wave's packed rows of block j into stage j mod (PD - 1) of its region
+    auto wbase = [&](int j) __attribute__((always_inline)) {
+        return uint32_t(C::OFF_W + (wid * (C::PD - 1) + (C::PD > 2 ? j % (C::PD - 1) : 0)) * C::WREG);
+    };
     uint32_t wo[C::NWW];
 #pragma unroll
     for (int s = 0; s < C::NWW; ++s) {
@@ -97,11 +103,11 @@ __global__ __launch_bounds__(64 * C::NW, C::WPS) void wslab_kernel(MatGroup grp,
         for (int s = 0; s < C::NWW; ++s) {
             if ((s + 1) * 64 > C::WSU && s * 64 + lane >= C::WSU) continue;
             if constexpr (C::ALIGNED) {
-                dma16s(rw, wo[s], uint32_t(j) * uint32_t(C::SB), lds0 + wbase + uint32_t(s * 1024));
+                dma16s(rw, wo[s], uint32_t(j) * uint32_t(C::SB), lds0 + wbase(j) + uint32_t(s * 1024));
             } else {
                 const int p = s * 64 + lane, pc = p - p / C::WCR * C::WCR;
                 dma16s(rw, ((wo[s] + uint32_t(j) * uint32_t(C::SB)) & ~15u) + 16u * uint32_t(pc), 0u,
-                       lds0 + wbase + uint32_t(s * 1024));
+                       lds0 + wbase(j) + uint32_t(s * 1024));
             }
         }
     };
@@ -140,30 +146,36 @@ __global__ __launch_bounds__(64 * C::NW, C::WPS) void wslab_kernel(MatGroup grp,
         }
     };
     SlabB B;
-    // waits for all of this wave's transfers (block j's rows among them)
+    // waits for this wave's transfers of block j: the PD - 2 blocks after it may
+    // be in flight (retired in order; near the end fewer were issued: all)
     auto decode = [&](int j) __attribute__((always_inline)) {
-        wait_vmcnt<0>();
+        if (C::PD > 2 && j + C::PD - 2 < nbk) wait_vmcnt<(C::PD - 2) * C::L>();
+        else wait_vmcnt<0>();
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
         const uint32_t mis =
             C::ALIGNED ? 0u : (uint32_t(16 * wid + nl) * uint32_t(a.row_bytes) + bl + uint32_t(j) * uint32_t(C::SB)) & 15u;
-        slab_unpack<F>(lds + wbase + nl * (C::WCR * 16) + mis, cl, B);
+        slab_unpack<F>(lds + wbase(j) + nl * (C::WCR * 16) + mis, cl, B);
     };
 
     f32x4v acc[TT];
 #pragma unroll
     for (int t = 0; t < TT; ++t) acc[t] = f32x4v{};
 
-    issue_w(0);
-    issue_a(0, 0);
+#pragma unroll
+    for (int p = 0; p + 1 < C::PD; ++p)
+        if (p < nbk) {
+            issue_w(p);
+            issue_a(p, p);
+        }
     decode(0);
     lds_barrier();
     for (int j = 0; j < nbk; ++j) {
-        if (j + 1 < nbk) {
-            issue_w(j + 1);
-            issue_a(j + 1, (j + 1) & 1);
+        if (j + C::PD - 1 < nbk) {
+            issue_w(j + C::PD - 1);
+            issue_a(j + C::PD - 1, (j + C::PD - 1) % C::PD);
         }
-        const uint8_t *sb = lds + (j & 1) * C::STAGE;
+        const uint8_t *sb = lds + (j % C::PD) * C::STAGE;
         const uint8_t *sa = sb + 16 * lane;
         const uint8_t *sm = sb + C::OFF_B + 8 * lane;
         const uint8_t *sd = sb + C::OFF_D + 16 * cl;
@@ -205,7 +217,7 @@ __global__ __launch_bounds__(64 * C::NW, C::WPS) void wslab_kernel(MatGroup grp,
             };
             load_a(0, 0);
             load_d(0, 0);
-            load_a(1, 1);
+            if (TT > 1) load_a(1, 1);
             mm(0);
 #pragma unroll
             for (int t = 0; t < TT; ++t) {
@@ -227,7 +239,7 @@ __global__ __launch_bounds__(64 * C::NW, C::WPS) void wslab_kernel(MatGroup grp,
         }
         if (j + 1 < nbk) {
             decode(j + 1);
-            lds_barrier();  // every wave's transfers of block j + 1 have landed, and stage j & 1 is free
+            lds_barrier();  // every wave's transfers of block j + 1 have landed, and stage j % PD is free
         }
     }
 
@@ -306,9 +318,42 @@ hipError_t launch_wslab(const WslabPlan &p, const MatArgs *tasks, int n, const Q
     if (p.shape == 'B') return launch_wslab_t<WsCfg<F, 4, 8, 4>, F>(tasks, n, x, s);
     return launch_wslab_t<WsCfg<F, 4, 4, 3>, F>(tasks, n, x, s);
 }
+// Up to 64 tokens: one group of all the tokens, 64 rows in 4 waves, three
+// stages (two blocks in flight: a block's work is short). The small-M kernels
+// read every token's codes again for each 16 rows (at 16-row tiles about 12
+// TB/s out of the L2s, their bound) and again the rows for each token group;
+// here 64 rows share them. Measured (K = 2560 unless said, us, small-M kernel
+// -> this): M = 48 at 19456 / 30000 / 100000 rows Q4_K 23.4 / 32.6 / 98.7 ->
+// 21.1 / 22.1 / 68.7, Q6_K 27.3 / 40.7 / 121 -> 25.3 / 27.3 / 81.9, Q5_K 30000
+// x 4096 57.2 -> 36.3; M = 64 Q4_K 24.1 / 34.0 / 102 -> 23.5 / 24.7 / 74.3.
+// Under one workgroup per CU (9728 rows at M = 37..64: 12.2..16 against
+// 15.3..19) a step's latency shows and the small-M kernels stay. At 17..32
+// tokens they take each 16-row tile's tokens at once: faster here only for
+// Q4_K from 7/4 workgroups per CU (30000 / 100000 rows 20.6 / 55.2 -> 18.3 /
+// 48.9). At 9..16 tokens Q6_K alone gains (decoding bound, one stage pair and
+// four waves per SIMD): 151936 rows 82 -> 79, 100000 x 4096 97 -> 86.
+template <class F>
+hipError_t launch_wslab_tall(const MatArgs *tasks, int n, const Q8KView &x, hipStream_t s) {
+    const int M = tasks[0].M, cus = mfma_cu_count();
+    int s64 = 0;
+    for (int i = 0; i < n; ++i) s64 += (tasks[i].N + 63) / 64;
+    if (M <= 8 || M > 64 || s64 < cus || !slab_ok<F>(tasks, n, x)) return hipErrorNotSupported;
+    // (Q5_K and Q6_K gain less: a few CUs with a second workgroup undo it, 16400
+    // rows at M = 60 25.9 against 27.0)
+    if (M > 32 && !std::is_same_v<F, MQ4KS> && s64 > cus && 8 * s64 < 9 * cus) return hipErrorNotSupported;
+    if (M > 48) return launch_wslab_t<WsCfg<F, 4, 4, 2, 3>, F>(tasks, n, x, s);
+    if (M > 32) return launch_wslab_t<WsCfg<F, 3, 4, 2, 3>, F>(tasks, n, x, s);
+    if constexpr (std::is_same_v<F, MQ4KS>)
+        if (M > 16 && 4 * s64 >= 7 * cus) return launch_wslab_t<WsCfg<F, 2, 4, 3, 3>, F>(tasks, n, x, s);
+    if constexpr (std::is_same_v<F, MQ6KS>)
+        if (M <= 16 && s64 >= 4 * cus) return launch_wslab_t<WsCfg<F, 1, 4, 4, 2>, F>(tasks, n, x, s);
+    return hipErrorNotSupported;
+}
+
 #define QMM_WSLAB(F)                                             \
     template WslabPlan wslab_plan<F>(const MatArgs *, int);      \
-    template hipError_t launch_wslab<F>(const WslabPlan &, const MatArgs *, int, const Q8KView &, hipStream_t);
+    template hipError_t launch_wslab<F>(const WslabPlan &, const MatArgs *, int, const Q8KView &, hipStream_t); \
+    template hipError_t launch_wslab_tall<F>(const MatArgs *, int, const Q8KView &, hipStream_t);
 QMM_WSLAB(MQ4KS)
 QMM_WSLAB(MQ5KS)
 QMM_WSLAB(MQ6KS)

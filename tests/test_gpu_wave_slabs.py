@@ -47,7 +47,17 @@ def test_wave_slabs(ctx, oracle, type_id, rows, K, M, residual):
     _run(ctx, oracle, type_id, rows, K, M, residual)
 
 
-@pytest.mark.parametrize("rows,K,M", [([5000], 768, 1000), ([6000], 256, 600), ([9000], 768, 300)])
+@pytest.mark.parametrize("type_id,rows,K,M,residual", [
+    # 64 rows x 64, 48, 32 and 16 tokens: one block (fewer than the stages), two, three and more; ragged tokens and rows
+    (TYPE_Q4_K, [16400], 256, 64, True), (TYPE_Q5_K, [20001], 512, 50, False), (TYPE_Q6_K, [19000], 768, 49, False),
+    (TYPE_Q4_K, [9728, 9700], 1280, 37, True), (TYPE_Q5_K, [19456], 256, 48, False), (TYPE_Q6_K, [20003], 512, 33, True),
+    (TYPE_Q4_K, [30000], 768, 17, False), (TYPE_Q4_K, [29001], 256, 32, True),
+    (TYPE_Q6_K, [65600], 256, 9, True), (TYPE_Q6_K, [65537], 768, 16, False)])
+def test_wave_slabs_tall(ctx, oracle, type_id, rows, K, M, residual):
+    _run(ctx, oracle, type_id, rows, K, M, residual)
+
+
+@pytest.mark.parametrize("rows,K,M", [([20000], 768, 40), ([66000], 768, 12), ([5000], 768, 1000), ([6000], 256, 600), ([9000], 768, 300)])
 def test_wave_slabs_unaligned_q6k(ctx, oracle, rows, K, M):
     """Q6_K rows from row 1 of a tensor: 210-B blocks 2 B off a 4-B boundary."""
     _run(ctx, oracle, TYPE_Q6_K, rows, K, M, False, skip=1)
