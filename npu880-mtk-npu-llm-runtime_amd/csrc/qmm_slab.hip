@@ -841,7 +841,8 @@ hipError_t launch_slab(const MatArgs *tasks, int n, const typename ActOf<F>::T &
         return hipErrorNotSupported;
     }
     // Past 64 tokens: the wave slabs (qmm_wslab.hip) where their expected time
-    // per block is at least 8 % below that of this file's kernels, which win
+    // per block is at least 8 % below that of this file's kernels of 32 and 128
+    // tokens (or below that of 256 tokens at all), which win
     // where the workgroups are few (their steps are shorter, their tiles
     // smaller). Their times per block, fitted over the same sweep with w
     // workgroups per CU and a call's fixed 4 us taken off: decoded slabs Q6_K
@@ -865,14 +866,26 @@ hipError_t launch_slab(const MatArgs *tasks, int n, const typename ActOf<F>::T &
     }
     const int t128 = (a.M + 127) / 128, t32 = (a.M + 31) / 32;
     const bool decoded = std::is_same_v<F, MQ6KS> || (std::is_same_v<F, MQ5KS> && 8 * w32 * t128 >= 5 * cus);
-    const int64_t ns = std::is_same_v<F, MQ6KS> ? 100 + int64_t(560) * w16 * t128 / cus
+    // Q6_K also 32 rows x 256 tokens in 8 waves, two-deep steps (each block
+    // decoded once per 256 tokens, one workgroup per CU): 1.3 us a block while
+    // they make one round, 1.45 a round after that (2560 x 9728 at M = 512:
+    // 55.6 -> 52.3 us, 4096 x 4096 at M = 512 35.5 -> 27.5; at M = 333, half
+    // its tokens unused, 52.5 against 42.8; 5000 x 5120 at M = 400 61 against 51).
+    const int r256 = (w32 * ((a.M + 255) / 256) + cus - 1) / cus;
+    const int64_t ns256 = r256 == 1 ? 1300 : 1450 * int64_t(r256);
+    const int64_t ns128 = std::is_same_v<F, MQ6KS> ? 100 + int64_t(560) * w16 * t128 / cus
                        : decoded                ? 300 + int64_t(920) * w32 * t128 / cus
                                                 : 350 + int64_t(500) * w64 * t32 / cus;
+    const bool wide = std::is_same_v<F, MQ6KS> && 100 * ns256 < 95 * ns128;
+    const int64_t ns = wide ? ns256 : ns128;
     const WslabPlan plan = wslab_plan<F>(tasks, n);
-    if (108 * plan.ns < 100 * ns) return launch_wslab<F>(plan, tasks, n, x, s);
+    if ((wide ? 100 : 108) * plan.ns < 100 * ns) return launch_wslab<F>(plan, tasks, n, x, s);
     if (decoded) {
         hipError_t e = hipErrorNotSupported;
-        if constexpr (std::is_same_v<F, MQ6KS>) e = launch_dslab_t<DsCfg<F, 1, 4, 2>, F>(tasks, n, x, s);
+        if constexpr (std::is_same_v<F, MQ6KS>) {
+            if (wide) e = launch_dslab_t<DsCfg<F, 2, 8, 2, 2, 3, 1, true>, F>(tasks, n, x, s);
+            if (e == hipErrorNotSupported) e = launch_dslab_t<DsCfg<F, 1, 4, 2>, F>(tasks, n, x, s);
+        }
         if constexpr (std::is_same_v<F, MQ5KS>) e = launch_dslab_t<DsCfg<F, 2, 4, 2>, F>(tasks, n, x, s);
         if (e != hipErrorNotSupported) return e;  // (its scales past the LDS: the packed slabs)
     }

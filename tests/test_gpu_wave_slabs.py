@@ -47,6 +47,14 @@ def test_wave_slabs(ctx, oracle, type_id, rows, K, M, residual):
     _run(ctx, oracle, type_id, rows, K, M, residual)
 
 
+@pytest.mark.parametrize("rows,K,M,residual", [([4096], 4352, 512, False), ([2003], 4608, 1000, True),
+                                               ([6100, 900], 4352, 250, False)])
+def test_decoded_slabs_256_tokens(ctx, oracle, rows, K, M, residual):
+    """Q6_K decoded slabs of 32 rows x 256 tokens (csrc/qmm_slab.hip), where
+    they make one round: odd and even step counts, ragged rows and tokens."""
+    _run(ctx, oracle, TYPE_Q6_K, rows, K, M, residual)
+
+
 @pytest.mark.parametrize("type_id,rows,K,M,residual", [
     # 64 rows x 64, 48, 32 and 16 tokens: one block (fewer than the stages), two, three and more; ragged tokens and rows
     (TYPE_Q4_K, [16400], 256, 64, True), (TYPE_Q5_K, [20001], 512, 50, False), (TYPE_Q6_K, [19000], 768, 49, False),
