@@ -7,6 +7,7 @@
 // id = 127.0f / amax correctly rounded, q = rint(x * id) (round to nearest
 // even, as lrintf under the default mode), clamp to [-127, 127].
 #include "qmm_device.h"
+#include "qmm_route.h"
 
 namespace qmm {
 
@@ -150,10 +151,11 @@ __global__ __launch_bounds__(256) void rmsnorm_q8k_kernel(const float *__restric
                                                           float *__restrict__ y, Q8KOut o) {
     __shared__ float part[4];
     const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
-    // per > 0: `per` consecutive rows (whole token tiles) on each XCD, whose
-    // L2 then merges the 16 rows' interleaved pieces of the tiles section
-    const size_t m = per ? size_t(blockIdx.x % 8u) * size_t(per) + blockIdx.x / 8u : blockIdx.x;
-    if (m >= size_t(M)) return;
+    // per > 0: `per` consecutive rows on each XCD, whose L2 then merges the 16
+    // rows' interleaved pieces of a token tile in the tiles section
+    const int row = xcd_row(blockIdx.x, per);
+    if (row >= M) return;
+    const size_t m = size_t(row);
     const float *xr = x + m * size_t(K);
     const int nq = K >> 2;  // float4s in the row
     // every load of the row and the weights is requested before the sum waits
@@ -309,8 +311,7 @@ hipError_t launch_rmsnorm_q8k(const float *x, const float *gamma, int M, int K, 
                               void *out, hipStream_t s) {
     const Q8KOut o = q8k_out(out, M, K);
     const int nj = (K / 4 + 255) / 256;  // float4s per thread
-    // from 16 token tiles on, two or more for each XCD; fewer rows spread over all of them
-    const int per = M >= 256 ? ((M + 15) / 16 + 7) / 8 * 16 : 0;
+    const int per = rms_rows_per_xcd(M);
     const unsigned grid = per ? unsigned(8 * per) : unsigned(M);
 #define QMM_RMS(NJ) \
     hipLaunchKernelGGL(rmsnorm_q8k_kernel<NJ>, dim3(grid), dim3(256), 0, s, x, gamma, M, K, per, y, o)

@@ -1,0 +1,32 @@
+// Prints what csrc/qmm_route.h decides for each line of stdin (tests/test_route.py).
+#include <cstdio>
+#include <cstring>
+#include <vector>
+
+#include "qmm_route.h"
+
+int main() {
+    char what[32];
+    while (std::scanf("%31s", what) == 1) {
+        if (!std::strcmp(what, "rms_rows")) {  // M: rows on each XCD, rows missed or taken twice
+            int M;
+            if (std::scanf("%d", &M) != 1) return 1;
+            const int per = qmm::rms_rows_per_xcd(M), grid = per ? 8 * per : M;
+            std::vector<int> seen(M), xcd(8);
+            int bad = 0;
+            for (int b = 0; b < grid; ++b) {
+                const int m = qmm::xcd_row(unsigned(b), per);
+                if (m >= M) continue;
+                ++seen[m];
+                ++xcd[b % 8];
+            }
+            for (int m = 0; m < M; ++m) bad += seen[m] != 1;
+            std::printf("%d", bad);
+            for (int x : xcd) std::printf(" %d", x);
+            std::printf("\n");
+        } else {
+            return 1;
+        }
+    }
+    return 0;
+}

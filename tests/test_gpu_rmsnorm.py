@@ -5,7 +5,7 @@ bit-exact), and against the oracle's own codes wherever y agrees."""
 import numpy as np
 import pytest
 
-from gpu_util import say
+from gpu_util import check_q8k, say
 
 pytestmark = pytest.mark.gpu
 
@@ -39,6 +39,32 @@ def test_rmsnorm_q8k(ctx, oracle, M, K):
     # and equal to the oracle's own codes in every block where y agrees
     same = (y == ry).reshape(M, K // 256, 256).all(axis=2)
     assert np.array_equal(qs.reshape(M, -1, 256)[same], rqs.reshape(M, -1, 256)[same])
+    for b in (xb, gb, yb, q):
+        ctx.free(b)
+
+
+@pytest.mark.parametrize("M,K", [(255, 256), (256, 2560), (257, 1280), (272, 4352), (300, 2560), (520, 512),
+                                 (1000, 256)])
+def test_rmsnorm_rows_over_xcds(ctx, oracle, M, K):
+    """Rows placed on the XCDs in consecutive eighths (M >= 256) and one by one
+    below: every row written once, ragged last eighth and token tile, every
+    section of the output. The output starts as bytes that no result has."""
+    say(f"rmsnorm rows M={M} K={K}")
+    g = np.random.default_rng(M + K)
+    x = (g.standard_normal((M, K)) * 3).astype(np.float32)
+    gamma = g.uniform(0.5, 1.5, K).astype(np.float32)
+    xb, gb = ctx.upload(x), ctx.upload(gamma)
+    yb = ctx.upload(np.full((M, K), np.nan, np.float32))
+    q = ctx.upload(np.full(int(ctx.lib.qmm_q8k_bytes(M, K)), 0xA5, np.uint8))
+    ctx.rmsnorm_q8k(xb, gb, M, K, yb, q)
+    ctx.sync()
+    y = ctx.d2h(yb, np.float32, (M, K))
+    ry, _ = oracle.rmsnorm_q8k(x, gamma)
+    # y: fp16 values; the order of the sum moves inv_rms by a few fp32 ulps, so
+    # a value that lies on a rounding boundary by one fp16 ulp (2^-10 relative)
+    assert np.all(np.abs(y - ry) <= np.maximum(np.abs(ry), 6.1e-5) * 2.0 ** -10)
+    assert np.mean(y != ry) < 0.01
+    check_q8k(ctx, oracle, q, M, K, y)
     for b in (xb, gb, yb, q):
         ctx.free(b)
 
