@@ -160,13 +160,18 @@ __global__ __launch_bounds__(256) void rmsnorm_q8k_kernel(const float *__restric
     const int nq = K >> 2;  // float4s in the row
     // every load of the row and the weights is requested before the sum waits
     // for its own (rows of 2560, M = 1 / 512 / 2048, with the register
-    // reductions: 4.7 / 7.3 / 14.8 -> 3.8 / 5.5 / 12.1 us)
+    // reductions, graph-timed: 4.5 / 7.1 / 15.9 -> 3.5 / 5.9 / 12.8 us). Past
+    // 10240 columns the weights wait until after the sum: held beside the row
+    // they take 172 registers, two workgroups per CU instead of four (rows of
+    // 12288, M = 37 / 520 / 2048: 14.5 / 22.5 / 77.6 before, 10.5 / 23.9 /
+    // 84.2 with them ahead, 11.0 / 21.3 / 65.2 so)
+    constexpr bool kAhead = NJ <= 10;
     float4 h[NJ], g[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
         const int q = min(t + 256 * j, nq - 1);  // (a thread past the row repeats its last values, unused)
         h[j] = reinterpret_cast<const float4 *>(xr)[q];
-        g[j] = reinterpret_cast<const float4 *>(gamma)[q];
+        if (kAhead) g[j] = reinterpret_cast<const float4 *>(gamma)[q];
     }
     // the sum of squares in the batch-1 activation fill's layout (so the GEMV
     // that normalizes its own input forms the same inv_rms)
@@ -187,6 +192,7 @@ __global__ __launch_bounds__(256) void rmsnorm_q8k_kernel(const float *__restric
         const int q = t + 256 * j;
         if (4 * (256 * j + 64 * wid) >= K) break;  // whole waves past the row's end
         float4 r;
+        if (!kAhead) g[j] = reinterpret_cast<const float4 *>(gamma)[q];
         r.x = round_to_fp16(round_to_fp16(h[j].x) * inv_rms * round_to_fp16(g[j].x));  // E:4301
         r.y = round_to_fp16(round_to_fp16(h[j].y) * inv_rms * round_to_fp16(g[j].y));
         r.z = round_to_fp16(round_to_fp16(h[j].z) * inv_rms * round_to_fp16(g[j].z));

@@ -10,7 +10,7 @@ from gpu_util import check_q8k, say
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("M,K", [(1, 256), (1, 2560), (4, 4096), (3, 9728), (2, 16384)])
+@pytest.mark.parametrize("M,K", [(1, 256), (1, 2560), (4, 4096), (3, 9728), (2, 16384), (3, 10240), (2, 10496)])
 def test_rmsnorm_q8k(ctx, oracle, M, K):
     say(f"rmsnorm_q8k M={M} K={K}")
     g = np.random.default_rng(M * 7 + K)
@@ -44,7 +44,7 @@ def test_rmsnorm_q8k(ctx, oracle, M, K):
 
 
 @pytest.mark.parametrize("M,K", [(255, 256), (256, 2560), (257, 1280), (272, 4352), (300, 2560), (520, 512),
-                                 (1000, 256)])
+                                 (1000, 256), (300, 10496)])
 def test_rmsnorm_rows_over_xcds(ctx, oracle, M, K):
     """Rows placed on the XCDs in consecutive eighths (M >= 256) and one by one
     below: every row written once, ragged last eighth and token tile, every
