@@ -111,18 +111,14 @@ __global__ __launch_bounds__(256) void quantize_q8_0_kernel(const float *__restr
 }
 
 // swiglu_chunk_worker (E:4349-4357): h = silu_mul(gate, up) per value, then
-// the fp16 round + Q8_K quantizer per 256-value block. Workgroups placed by
-// token tile as above (N = 9728 at M = 512 / 2048: 18.0 / 64.5 -> 15.6 / 60.0
-// us, 5.3 TB/s of the bytes it must move).
+// the fp16 round + Q8_K quantizer per 256-value block, a wave each. Bound by
+// memory (9728 columns at M = 2048: 60.5 us, 5.3 TB/s of the bytes it must
+// move); workgroups placed by xcd_quad.
 __global__ __launch_bounds__(256) void swiglu_q8k_kernel(const float *__restrict__ gate,
-                                                         const float *__restrict__ up, int M, int nb, int nq, int total,
+                                                         const float *__restrict__ up, int M, int nb, int nq,
                                                          float *__restrict__ h, Q8KOut o) {
-    const int per = (int(gridDim.x) + 7) / 8;
-    const int lin = int(blockIdx.x % 8u) * per + int(blockIdx.x / 8u);
-    if (lin >= total) return;
-    const int mi = lin & 15, un = lin >> 4;
-    const int t = un / nq, q = un - t * nq;
-    const int m = 16 * t + mi, j = 4 * q + int(threadIdx.x >> 6);
+    const QuadItem it = xcd_quad(blockIdx.x, nq);
+    const int m = it.m, j = 4 * it.q + int(threadIdx.x >> 6);
     if (m >= M || j >= nb) return;
     const size_t blk = size_t(m) * size_t(nb) + size_t(j);
     const int lane = threadIdx.x & 63;
@@ -307,9 +303,9 @@ hipError_t launch_quantize_q8_0(const float *x, int M, int K, void *out, hipStre
 
 hipError_t launch_swiglu_q8k(const float *gate, const float *up, int M, int N, float *h,
                              void *out, hipStream_t s) {
-    const int nb = N / 256, nq = (nb + 3) / 4, total = ((M + 15) / 16) * nq * 16;
-    hipLaunchKernelGGL(swiglu_q8k_kernel, dim3(unsigned((total + 7) / 8 * 8)), dim3(256), 0, s, gate, up, M, nb, nq,
-                       total, h, q8k_out(out, M, N));
+    const int nb = N / 256, nq = (nb + 3) / 4;
+    hipLaunchKernelGGL(swiglu_q8k_kernel, dim3(xcd_quad_grid(M, nq)), dim3(256), 0, s, gate, up, M, nb, nq, h,
+                       q8k_out(out, M, N));
     return hipGetLastError();
 }
 

@@ -24,6 +24,22 @@ int main() {
             std::printf("%d", bad);
             for (int x : xcd) std::printf(" %d", x);
             std::printf("\n");
+        } else if (!std::strcmp(what, "quads")) {  // M, quads: items missed or taken twice, workgroups with work on each XCD
+            int M, nq;
+            if (std::scanf("%d %d", &M, &nq) != 2) return 1;
+            std::vector<int> seen(size_t(M) * nq), xcd(8);
+            int bad = 0;
+            for (unsigned b = 0; b < qmm::xcd_quad_grid(M, nq); ++b) {
+                const qmm::QuadItem it = qmm::xcd_quad(b, nq);
+                if (it.m >= M) continue;
+                if (it.q < 0 || it.q >= nq) return 1;
+                ++seen[size_t(it.m) * nq + it.q];
+                ++xcd[b % 8];
+            }
+            for (int v : seen) bad += v != 1;
+            std::printf("%d", bad);
+            for (int x : xcd) std::printf(" %d", x);
+            std::printf("\n");
         } else {
             return 1;
         }

@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 
 import synth
-from gpu_util import say
+from gpu_util import check_q8k, say
 from oracle import TYPE_Q4_K, TYPE_Q5_K, TYPE_Q6_K, TYPE_Q8_0
 
 pytestmark = pytest.mark.gpu
@@ -82,6 +82,28 @@ def test_swiglu_requant(ctx, oracle):
     assert np.array_equal(ctx.read_q8k_bh(out, M, N),
                           qs.reshape(M, N // 16, 16).astype(np.int32).sum(axis=2).astype(np.float32))
     assert np.array_equal(ctx.read_q8k_h(out, M, N), oracle.f32_to_fp16(h))
+    for b in (gb, ub, hb, out):
+        ctx.free(b)
+
+
+@pytest.mark.parametrize("M,N", [(1, 1280), (7, 1024), (8, 256), (15, 2560), (16, 1024), (17, 2304), (37, 2048),
+                                 (300, 1280)])
+def test_swiglu_tokens_and_quads(ctx, oracle, M, N):
+    """Ragged units of 8 tokens and quads of blocks: every row and block written,
+    every section. The outputs start as bytes that no result has."""
+    say(f"swiglu tokens M={M} N={N}")
+    g = synth.activations(M, N, seed=M + N) * 3
+    u = synth.activations(M, N, seed=M + N + 1)
+    gb, ub = ctx.upload(g), ctx.upload(u)
+    hb = ctx.upload(np.full((M, N), np.nan, np.float32))
+    out = ctx.upload(np.full(int(ctx.lib.qmm_q8k_bytes(M, N)), 0xA5, np.uint8))
+    ctx.swiglu_q8k(gb, ub, M, N, hb, out)
+    ctx.sync()
+    h = ctx.d2h(hb, np.float32, (M, N))
+    # SiLU uses the device expf: values within a few ulp of the host libm's
+    eh, _ = oracle.swiglu_q8k(g, u)
+    assert np.allclose(h, eh, rtol=1e-5, atol=1e-30)
+    check_q8k(ctx, oracle, out, M, N, h)
     for b in (gb, ub, hb, out):
         ctx.free(b)
 

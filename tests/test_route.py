@@ -34,3 +34,13 @@ def test_rmsnorm_rows_cover_and_balance(route):
         bad, *xcd = map(int, line.split())
         assert bad == 0 and sum(xcd) == M, (M, line)
         assert max(xcd) <= (M + 7) // 8, (M, xcd)
+
+
+def test_swiglu_quads_cover_and_balance(route):
+    """Every token's every quad once; the XCDs' workgroups differ by at most one
+    unit of 8 tokens and one ragged unit."""
+    cases = [(M, nq) for M in (1, 7, 8, 9, 15, 16, 17, 37, 65, 100, 257, 300, 513, 2048) for nq in (1, 3, 10, 14)]
+    for (M, nq), line in zip(cases, route([f"quads {M} {nq}" for M, nq in cases])):
+        bad, *xcd = map(int, line.split())
+        assert bad == 0 and sum(xcd) == M * nq, (M, nq, line)
+        assert max(xcd) - min(xcd) <= 8 + M % 8, (M, nq, xcd)
