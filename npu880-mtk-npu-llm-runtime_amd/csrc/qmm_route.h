@@ -1,7 +1,9 @@
-// qmm_route.h — which rows a producer's workgroup takes, as plain C++ (no
-// HIP): the kernels and launchers use these rules, and a host program can
-// check them without a device.
+// qmm_route.h — which rows a producer's workgroup takes, and which kernel a
+// GEMM of k-quant rows takes, as plain C++ (no HIP): the kernels and launchers
+// use these rules, and a host program can check them without a device.
 #pragma once
+
+#include <cstdint>
 
 namespace qmm {
 
@@ -34,5 +36,87 @@ constexpr QuadItem xcd_quad(unsigned b, int nq) {
     return QuadItem{u / nq * 8 + (i & 7), u % nq};
 }
 constexpr unsigned xcd_quad_grid(int M, int nq) { return unsigned(((M + 7) / 8 * nq + 7) / 8 * 64); }
+
+enum class KFormat { Q4, Q5, Q6 };
+
+// a task group's row tiles of 16, 32, 64 and 128 rows (each task rounded up)
+struct RowTiles {
+    int r16 = 0, r32 = 0, r64 = 0, r128 = 0;
+    void add(int rows) {
+        r16 += (rows + 15) / 16;
+        r32 += (rows + 31) / 32;
+        r64 += (rows + 63) / 64;
+        r128 += (rows + 127) / 128;
+    }
+};
+
+// Past 64 tokens. Wave slabs (qmm_wslab.hip) of 128 rows x 96 tokens, 128 x 64
+// and 64 x 64; decoded slabs (qmm_slab.hip) of 128 tokens (16 rows for Q6_K,
+// 32 for Q5_K) and, for Q6_K, of 32 rows x 256 tokens; packed slabs of 64 x 32.
+enum class Prefill : char { W128x96 = 'A', W128x64 = 'B', W64x64 = 'C', D128 = 'D', D256 = 'E', P64x32 = 'P' };
+
+// The kernel with the least expected time per 256-value block, in nanoseconds.
+// Wave slabs: a CU takes its share of the workgroups, rounded up; of the 8-wave
+// shapes two run side by side, and one left alone takes 0.7 of a pair's time
+// (64 x 64: its step has a floor that three side by side hide). A workgroup's
+// time per block, a call's fixed 4 us taken off, from a sweep of 18 shapes (M =
+// 192..2048). Measured (us, 128 x 96 / 128 x 64 / 64 x 64, chosen first): Q4_K
+// 2 x 9728 x 2560 at M = 2048 264 / 272 / 303, at M = 512 (128 x 64) 75 / 70 /
+// 75, at M = 192 (128 x 64) 40 / 32 / 36; 2560 x 4096 at M = 2048 60 / 63 / 66;
+// Q5_K 6144 x 2560 at M = 2048 (128 x 64) 105 / 102 / 113, at M = 512 (64 x 64)
+// 42 / 33 / 30; Q6_K 2560 x 9728 at M = 2048 156 / 187 / 186, 9728 x 2560 at M
+// = 512 47 / 54 / 49.
+// They are taken where that is at least 8 % below the slabs of 32 and 128
+// tokens (or below those of 256 at all), which win where the workgroups are few
+// (their steps are shorter, their tiles smaller). Fitted over the same sweep
+// with w workgroups per CU: decoded Q6_K 16 x 128 0.1 + 0.56 w us (2560 x 9728
+// at M = 512 / 1024 / 2048: 1.34 / 2.55 / 5.95), Q5_K 32 x 128 0.3 + 0.92 w
+// (6144 x 2560 at M = 200 / 512 / 2048: 1.7 / 2.9 / 11.5, 3001 x 8192 at M =
+// 777 2.6), packed 64 x 32 0.35 + 0.5 w (Q4_K 2560 x 4096 at M = 512 / 1024:
+// 1.3 / 2.5, 2 x 9728 x 2560 at M = 65: 1.9).
+// Q6_K and Q5_K decode in LDS (their decoding is costly next to their update)
+// from 65 tokens, Q5_K where those workgroups number at least 5/8 of the CUs
+// (QKV 6144 x 2560 at M = 65..127 17.4 -> 16.1 us; 4096 x 2560 at M = 128 12.8
+// against 16.2, 1024 x 2560 12.3 against 15.8 on the packed slabs: there they
+// stay). Q4_K stays packed: its update outweighs its decoding (2560 x 4096 at M
+// = 512 25.1 against 26.9 us and more).
+// Q6_K 32 x 256 (each block decoded once per 256 tokens, one workgroup per CU):
+// 1.3 us a block while they make one round, 1.45 a round after that, but a
+// longer start, so the time per block is not all. Over 8 heights, K = 512 /
+// 1024 / 2560 / 4096 / 9728 and M = 65..2048, against the 16 x 128 slabs: in
+// one round with w > 3 of those 0.89 / 0.86 / 0.77 / 0.73 / 0.66 of their time,
+// with 2 < w <= 3 1.15 / 1.12 / 1.07 / 1.04 / 0.88..1.04: there only over K >=
+// 8192 where their 128 tokens are in use (live: 2560 x 9728 at M = 512 52.8 ->
+// 51.7 us, 6144 x 9728 at M = 256 56.2 -> 52.1; 5000 x 5120 at M = 400 61
+// against 51); in several rounds 1.0..1.2 over K <= 1024.
+inline Prefill prefill_kernel(KFormat f, const RowTiles &r, int K, int M, int cus) {
+    const int i = int(f);
+    constexpr int k96[] = {1750, 2040, 2100}, k64[] = {1290, 1650, 1800}, kC[] = {780, 900, 960};
+    constexpr int kC0[] = {850, 1350, 1350}, kC1[] = {450, 400, 400};
+    auto load = [&](int wgs) { return (wgs + cus - 1) / cus; };
+    auto pairs = [&](int wgs, int64_t ns) {  // two per CU side by side
+        const int l = load(wgs);
+        return ns * (l & ~1) + (l & 1) * (ns * 27 / 20);
+    };
+    const int64_t a = pairs(r.r128 * ((M + 95) / 96), k96[i]), b = pairs(r.r128 * ((M + 63) / 64), k64[i]);
+    const int64_t lc = load(r.r64 * ((M + 63) / 64)), c0 = lc * kC[i], c1 = kC0[i] + lc * kC1[i], c = c0 > c1 ? c0 : c1;
+    const int64_t ab = b < a ? b : a, wave = c < ab ? c : ab;
+    const Prefill w = c < ab ? Prefill::W64x64 : b < a ? Prefill::W128x64 : Prefill::W128x96;
+
+    const int t16 = (M + 15) / 16, t32 = (M + 31) / 32, t128 = (M + 127) / 128;
+    const bool q6 = f == KFormat::Q6, decoded = q6 || (f == KFormat::Q5 && 8 * r.r32 * t128 >= 5 * cus);
+    const int64_t ns128 = q6        ? 100 + int64_t(560) * r.r16 * t128 / cus
+                          : decoded ? 300 + int64_t(920) * r.r32 * t128 / cus
+                                    : 350 + int64_t(500) * r.r64 * t32 / cus;
+    if (q6) {
+        const int rounds = load(r.r32 * ((M + 255) / 256));
+        const int64_t ns256 = rounds == 1 ? 1300 : 1450 * int64_t(rounds);
+        const int64_t live = int64_t(r.r16) * t16;  // (eight to a workgroup of 128 tokens)
+        const bool pays = rounds > 1 ? K >= 2048 : load(r.r16 * t128) > 3 || (K >= 8192 && 10 * live >= 8 * 24 * int64_t(cus));
+        if (pays && 100 * ns256 < 95 * ns128) return wave < ns256 ? w : Prefill::D256;
+    }
+    if (108 * wave < 100 * ns128) return w;
+    return decoded ? Prefill::D128 : Prefill::P64x32;
+}
 
 }  // namespace qmm

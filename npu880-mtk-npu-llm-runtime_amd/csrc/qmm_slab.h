@@ -3,6 +3,7 @@
 #pragma once
 
 #include "qmm_kformats.h"
+#include "qmm_route.h"
 
 namespace qmm {
 
@@ -82,14 +83,18 @@ inline bool slab_ok(const MatArgs *tasks, int n, const Q8KView &x) {
 template <class F>
 hipError_t launch_wslab_tall(const MatArgs *tasks, int n, const Q8KView &x, hipStream_t s);
 
-// the wave-slab shape of a call and its expected time per 256-value block
-struct WslabPlan {
-    char shape;
-    int64_t ns;
-};
+// a wave-slab shape (W128x96, W128x64 or W64x64)
 template <class F>
-WslabPlan wslab_plan(const MatArgs *tasks, int n);
+hipError_t launch_wslab(Prefill p, const MatArgs *tasks, int n, const Q8KView &x, hipStream_t s);
+
 template <class F>
-hipError_t launch_wslab(const WslabPlan &p, const MatArgs *tasks, int n, const Q8KView &x, hipStream_t s);
+constexpr KFormat kformat() {
+    return std::is_same_v<F, MQ4KS> ? KFormat::Q4 : std::is_same_v<F, MQ5KS> ? KFormat::Q5 : KFormat::Q6;
+}
+inline RowTiles row_tiles(const MatArgs *tasks, int n) {
+    RowTiles r;
+    for (int i = 0; i < n; ++i) r.add(tasks[i].N);
+    return r;
+}
 
 }  // namespace qmm

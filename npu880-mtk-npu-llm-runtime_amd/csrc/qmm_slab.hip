@@ -804,6 +804,7 @@ static hipError_t launch_slab_t(const MatArgs *tasks, int n, const typename ActO
 }
 
 int mfma_cu_count();
+
 // hipErrorNotSupported (nothing launched) where the slab kernels do not
 // apply (slab_ok), at 64 tokens or fewer outside the shapes below, or with a
 // decoded slab's LDS over the CU's.
@@ -840,55 +841,16 @@ hipError_t launch_slab(const MatArgs *tasks, int n, const typename ActOf<F>::T &
         }
         return hipErrorNotSupported;
     }
-    // Past 64 tokens: the wave slabs (qmm_wslab.hip) where their expected time
-    // per block is at least 8 % below that of this file's kernels of 32 and 128
-    // tokens (or below that of 256 tokens at all), which win
-    // where the workgroups are few (their steps are shorter, their tiles
-    // smaller). Their times per block, fitted over the same sweep with w
-    // workgroups per CU and a call's fixed 4 us taken off: decoded slabs Q6_K
-    // 16 x 128 0.1 + 0.56 w us (2560 x 9728 at M = 512 / 1024 / 2048: 1.34 /
-    // 2.55 / 5.95), Q5_K 32 x 128 0.3 + 0.92 w (6144 x 2560 at M = 200 / 512 /
-    // 2048: 1.7 / 2.9 / 11.5, 3001 x 8192 at M = 777 2.6), packed 64 x 32
-    // slabs 0.35 + 0.5 w (Q4_K 2560 x 4096 at M = 512 / 1024: 1.3 / 2.5, 2 x
-    // 9728 x 2560 at M = 65: 1.9).
-    // Q6_K and Q5_K decode in LDS (their decoding is costly next to their
-    // update) from 65 tokens, Q5_K where those workgroups number at least 5/8
-    // of the CUs (QKV 6144 x 2560 at M = 65..127 17.4 -> 16.1 us; 4096 x 2560
-    // at M = 128 12.8 against 16.2, 1024 x 2560 12.3 against 15.8 on the
-    // packed slabs: there they stay). Q4_K stays packed: its update outweighs
-    // its decoding (2560 x 4096 at M = 512 25.1 against 26.9 us and more).
-    const int cus = mfma_cu_count();
-    int w16 = 0, w32 = 0, w64 = 0;
-    for (int i = 0; i < n; ++i) {
-        w16 += (tasks[i].N + 15) / 16;
-        w32 += (tasks[i].N + 31) / 32;
-        w64 += (tasks[i].N + 63) / 64;
+    const Prefill p = prefill_kernel(kformat<F>(), row_tiles(tasks, n), a.K, a.M, mfma_cu_count());
+    if (p == Prefill::W128x96 || p == Prefill::W128x64 || p == Prefill::W64x64) return launch_wslab<F>(p, tasks, n, x, s);
+    hipError_t e = hipErrorNotSupported;  // (a decoded slab's scales past the LDS: the next kernel)
+    if constexpr (std::is_same_v<F, MQ6KS>) {
+        if (p == Prefill::D256) e = launch_dslab_t<DsCfg<F, 2, 8, 2, 2, 3, 1, true>, F>(tasks, n, x, s);
+        if (e == hipErrorNotSupported) e = launch_dslab_t<DsCfg<F, 1, 4, 2>, F>(tasks, n, x, s);
     }
-    const int t128 = (a.M + 127) / 128, t32 = (a.M + 31) / 32;
-    const bool decoded = std::is_same_v<F, MQ6KS> || (std::is_same_v<F, MQ5KS> && 8 * w32 * t128 >= 5 * cus);
-    // Q6_K also 32 rows x 256 tokens in 8 waves, two-deep steps (each block
-    // decoded once per 256 tokens, one workgroup per CU): 1.3 us a block while
-    // they make one round, 1.45 a round after that (2560 x 9728 at M = 512:
-    // 55.6 -> 52.3 us, 4096 x 4096 at M = 512 35.5 -> 27.5; at M = 333, half
-    // its tokens unused, 52.5 against 42.8; 5000 x 5120 at M = 400 61 against 51).
-    const int r256 = (w32 * ((a.M + 255) / 256) + cus - 1) / cus;
-    const int64_t ns256 = r256 == 1 ? 1300 : 1450 * int64_t(r256);
-    const int64_t ns128 = std::is_same_v<F, MQ6KS> ? 100 + int64_t(560) * w16 * t128 / cus
-                       : decoded                ? 300 + int64_t(920) * w32 * t128 / cus
-                                                : 350 + int64_t(500) * w64 * t32 / cus;
-    const bool wide = std::is_same_v<F, MQ6KS> && 100 * ns256 < 95 * ns128;
-    const int64_t ns = wide ? ns256 : ns128;
-    const WslabPlan plan = wslab_plan<F>(tasks, n);
-    if ((wide ? 100 : 108) * plan.ns < 100 * ns) return launch_wslab<F>(plan, tasks, n, x, s);
-    if (decoded) {
-        hipError_t e = hipErrorNotSupported;
-        if constexpr (std::is_same_v<F, MQ6KS>) {
-            if (wide) e = launch_dslab_t<DsCfg<F, 2, 8, 2, 2, 3, 1, true>, F>(tasks, n, x, s);
-            if (e == hipErrorNotSupported) e = launch_dslab_t<DsCfg<F, 1, 4, 2>, F>(tasks, n, x, s);
-        }
-        if constexpr (std::is_same_v<F, MQ5KS>) e = launch_dslab_t<DsCfg<F, 2, 4, 2>, F>(tasks, n, x, s);
-        if (e != hipErrorNotSupported) return e;  // (its scales past the LDS: the packed slabs)
-    }
+    if constexpr (std::is_same_v<F, MQ5KS>)
+        if (p == Prefill::D128) e = launch_dslab_t<DsCfg<F, 2, 4, 2>, F>(tasks, n, x, s);
+    if (e != hipErrorNotSupported) return e;
     // 64 rows x 32 tokens in 4 waves, three or four workgroups per CU (O 2560
     // x 4096 at M = 512: 28.5 -> 23.9 us against 64 x 64). Measured slower at
     // M = 512: 32 x 64, 64 x 16, 32 x 32, three stages, two row tiles per wave.

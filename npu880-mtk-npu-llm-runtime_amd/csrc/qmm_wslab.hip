@@ -274,50 +274,15 @@ static hipError_t launch_wslab_t(const MatArgs *tasks, int n, const Q8KView &x, 
 
 int mfma_cu_count();
 
-// The shapes: A 128 rows x 96 tokens and B 128 x 64 in 8 waves (two
-// workgroups per CU), C 64 x 64 in 4 waves (three per CU).
-//
-// WslabPlan: the shape with the least expected time per block, in
-// nanoseconds. A CU takes its share of the workgroups, rounded up; of the
-// 8-wave shapes two run side by side, and one left alone takes 0.7 of a
-// pair's time (C: its step has a floor that three side by side hide). ns: a
-// workgroup's time per block, a call's fixed 4 us taken off, from the sweep
-// of 18 shapes below (M = 192..2048). Measured (us, A / B / C, chosen first):
-// Q4_K 2 x 9728 x 2560 at M = 2048 264 / 272 / 303, at M = 512 (B) 75 / 70 /
-// 75, at M = 192 (B) 40 / 32 / 36; 2560 x 4096 at M = 2048 60 / 63 / 66; Q5_K
-// 6144 x 2560 at M = 2048 (B) 105 / 102 / 113, at M = 512 (C) 42 / 33 / 30;
-// Q6_K 2560 x 9728 at M = 2048 156 / 187 / 186, 9728 x 2560 at M = 512 47 /
-// 54 / 49.
+// 128 rows x 96 and 128 x 64 tokens in 8 waves (two workgroups per CU), 64 x
+// 64 in 4 waves (three per CU); prefill_kernel chooses.
 template <class F>
-WslabPlan wslab_plan(const MatArgs *tasks, int n) {
-    constexpr int kA = std::is_same_v<F, MQ4KS> ? 1750 : std::is_same_v<F, MQ5KS> ? 2040 : 2100;
-    constexpr int kB = std::is_same_v<F, MQ4KS> ? 1290 : std::is_same_v<F, MQ5KS> ? 1650 : 1800;
-    constexpr int kC = std::is_same_v<F, MQ4KS> ? 780 : std::is_same_v<F, MQ5KS> ? 900 : 960;
-    constexpr int kC0 = F::kMin && F::kShift == 3 ? 850 : 1350, kC1 = F::kMin && F::kShift == 3 ? 450 : 400;
-    int s128 = 0, s64 = 0;
-    for (int i = 0; i < n; ++i) {
-        s128 += (tasks[i].N + 127) / 128;
-        s64 += (tasks[i].N + 63) / 64;
-    }
-    const int M = tasks[0].M, cus = mfma_cu_count();
-    auto load = [&](int wgs) { return (wgs + cus - 1) / cus; };
-    auto pairs = [&](int wgs, int64_t ns) {  // two per CU side by side
-        const int l = load(wgs);
-        return ns * (l & ~1) + (l & 1) * (ns * 27 / 20);
-    };
-    const int64_t lc = load(s64 * ((M + 63) / 64));
-    const WslabPlan a{'A', pairs(s128 * ((M + 95) / 96), kA)}, b{'B', pairs(s128 * ((M + 63) / 64), kB)},
-        c{'C', std::max(lc * kC, kC0 + lc * kC1)};
-    const WslabPlan &m = b.ns < a.ns ? b : a;
-    return c.ns < m.ns ? c : m;
-}
-
-template <class F>
-hipError_t launch_wslab(const WslabPlan &p, const MatArgs *tasks, int n, const Q8KView &x, hipStream_t s) {
-    if (p.shape == 'A') return launch_wslab_t<WsCfg<F, 6, 8, 4>, F>(tasks, n, x, s);
-    if (p.shape == 'B') return launch_wslab_t<WsCfg<F, 4, 8, 4>, F>(tasks, n, x, s);
+hipError_t launch_wslab(Prefill p, const MatArgs *tasks, int n, const Q8KView &x, hipStream_t s) {
+    if (p == Prefill::W128x96) return launch_wslab_t<WsCfg<F, 6, 8, 4>, F>(tasks, n, x, s);
+    if (p == Prefill::W128x64) return launch_wslab_t<WsCfg<F, 4, 8, 4>, F>(tasks, n, x, s);
     return launch_wslab_t<WsCfg<F, 4, 4, 3>, F>(tasks, n, x, s);
 }
+
 // Up to 64 tokens: one group of all the tokens, 64 rows in 4 waves, three
 // stages (two blocks in flight: a block's work is short). The small-M kernels
 // read every token's codes again for each 16 rows (at 16-row tiles about 12
@@ -350,9 +315,8 @@ hipError_t launch_wslab_tall(const MatArgs *tasks, int n, const Q8KView &x, hipS
     return hipErrorNotSupported;
 }
 
-#define QMM_WSLAB(F)                                             \
-    template WslabPlan wslab_plan<F>(const MatArgs *, int);      \
-    template hipError_t launch_wslab<F>(const WslabPlan &, const MatArgs *, int, const Q8KView &, hipStream_t); \
+#define QMM_WSLAB(F)                                                                                     \
+    template hipError_t launch_wslab<F>(Prefill, const MatArgs *, int, const Q8KView &, hipStream_t); \
     template hipError_t launch_wslab_tall<F>(const MatArgs *, int, const Q8KView &, hipStream_t);
 QMM_WSLAB(MQ4KS)
 QMM_WSLAB(MQ5KS)

@@ -40,6 +40,15 @@ int main() {
             std::printf("%d", bad);
             for (int x : xcd) std::printf(" %d", x);
             std::printf("\n");
+        } else if (!std::strcmp(what, "prefill")) {  // format, K, M, CUs, tasks, rows of each: the kernel past 64 tokens
+            int f, K, M, cus, n;
+            if (std::scanf("%d %d %d %d %d", &f, &K, &M, &cus, &n) != 5) return 1;
+            qmm::RowTiles r;
+            for (int rows; n > 0; --n) {
+                if (std::scanf("%d", &rows) != 1) return 1;
+                r.add(rows);
+            }
+            std::printf("%c\n", char(qmm::prefill_kernel(qmm::KFormat(f - 4), r, K, M, cus)));
         } else {
             return 1;
         }

@@ -35,24 +35,32 @@ def _run(ctx, oracle, type_id, rows, K, M, residual, skip=0):
         ctx.free(b)
 
 
-@pytest.mark.parametrize("type_id,rows,K,M,residual", [
+# kernel (csrc/qmm_route.h): cases that take it at 256 CUs (tests/test_route.py checks that they do)
+PREFILL = {
     # 128 rows x 96 tokens: ragged last tokens (80, 40, 70 of 96) and rows
-    (TYPE_Q4_K, [3000], 512, 2000, True), (TYPE_Q6_K, [5001], 768, 1000, False), (TYPE_Q5_K, [4100], 256, 1030, True),
+    "A": [(TYPE_Q4_K, [3000], 512, 2000, True), (TYPE_Q6_K, [5001], 768, 1000, False), (TYPE_Q5_K, [4100], 256, 1030, True),
+          (TYPE_Q5_K, [6100], 256, 2000, False)],
     # 128 x 64
-    (TYPE_Q4_K, [5003], 768, 700, False), (TYPE_Q6_K, [6001], 512, 600, True), (TYPE_Q5_K, [6100], 256, 2000, False),
+    "B": [(TYPE_Q4_K, [5003], 768, 700, False), (TYPE_Q6_K, [6001], 512, 600, True), (TYPE_Q5_K, [6100], 256, 600, False),
+          (TYPE_Q5_K, [6020, 75], 512, 590, True)],
     # 64 x 64: one token past a group, a 49-row task in the group
-    (TYPE_Q4_K, [8190], 256, 257, True), (TYPE_Q5_K, [8201], 512, 300, False), (TYPE_Q6_K, [9001], 768, 300, False),
-    (TYPE_Q4_K, [2500, 49], 512, 1000, True)])
+    "C": [(TYPE_Q4_K, [8190], 256, 257, True), (TYPE_Q5_K, [8201], 512, 300, False), (TYPE_Q6_K, [9001], 768, 300, False),
+          (TYPE_Q4_K, [2500, 49], 512, 1000, True)],
+    # Q6_K decoded slabs of 32 rows x 256 tokens: odd and even step counts, ragged rows and tokens
+    "E": [(TYPE_Q6_K, [4096], 4352, 512, False), (TYPE_Q6_K, [2003], 4608, 1000, True),
+          (TYPE_Q6_K, [6100, 900], 4352, 250, False), (TYPE_Q6_K, [4090], 512, 509, True)],
+}
+
+
+@pytest.mark.parametrize("type_id,rows,K,M,residual", PREFILL["A"] + PREFILL["B"] + PREFILL["C"])
 def test_wave_slabs(ctx, oracle, type_id, rows, K, M, residual):
     _run(ctx, oracle, type_id, rows, K, M, residual)
 
 
-@pytest.mark.parametrize("rows,K,M,residual", [([4096], 4352, 512, False), ([2003], 4608, 1000, True),
-                                               ([6100, 900], 4352, 250, False)])
-def test_decoded_slabs_256_tokens(ctx, oracle, rows, K, M, residual):
-    """Q6_K decoded slabs of 32 rows x 256 tokens (csrc/qmm_slab.hip), where
-    they make one round: odd and even step counts, ragged rows and tokens."""
-    _run(ctx, oracle, TYPE_Q6_K, rows, K, M, residual)
+@pytest.mark.parametrize("type_id,rows,K,M,residual", PREFILL["E"])
+def test_decoded_slabs_256_tokens(ctx, oracle, type_id, rows, K, M, residual):
+    """Q6_K decoded slabs of 32 rows x 256 tokens (csrc/qmm_slab.hip)."""
+    _run(ctx, oracle, type_id, rows, K, M, residual)
 
 
 @pytest.mark.parametrize("type_id,rows,K,M,residual", [

@@ -1,10 +1,14 @@
-"""The rules of csrc/qmm_route.h (which rows a workgroup takes), through a small
-host program: no device needed."""
+"""The rules of csrc/qmm_route.h (which rows a workgroup takes, which kernel a GEMM
+takes), through a small host program: no device needed."""
 import os
 import subprocess
 
 import pytest
 
+from oracle import TYPE_Q4_K, TYPE_Q5_K, TYPE_Q6_K
+from test_gpu_wave_slabs import PREFILL
+
+FORMAT = {TYPE_Q4_K: 4, TYPE_Q5_K: 5, TYPE_Q6_K: 6}
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 PKG = os.path.join(ROOT, "npu880-mtk-npu-llm-runtime_amd")
 
@@ -44,3 +48,26 @@ def test_swiglu_quads_cover_and_balance(route):
         bad, *xcd = map(int, line.split())
         assert bad == 0 and sum(xcd) == M * nq, (M, nq, line)
         assert max(xcd) - min(xcd) <= 8 + M % 8, (M, nq, xcd)
+
+
+def _prefill(route, cases):
+    return route([f"prefill {FORMAT[t]} {K} {M} 256 {len(rows)} {' '.join(map(str, rows))}" for t, rows, K, M in cases])
+
+
+def test_prefill_kernels_of_the_gpu_cases(route):
+    """Each case of the wave-slab GPU tests takes the kernel it is there for."""
+    for kernel, cases in PREFILL.items():
+        assert _prefill(route, [c[:4] for c in cases]) == [kernel] * len(cases), kernel
+
+
+def test_prefill_q6k_256_tokens_only_where_faster(route):
+    """The 32 x 256 decoded slabs' longer start: in one round beside 2 to 3 of the
+    16 x 128 slabs per CU these were faster over short K (5000 x 512 at M = 192
+    6.2 against 7.2 us) and where half of 256 tokens are missing over long K."""
+    few = [([5000], 512, 192), ([2560], 512, 400), ([6144], 2560, 160), ([4096], 4096, 257), ([2560], 2560, 512),
+           ([5000], 9728, 160)]
+    assert set(_prefill(route, [(TYPE_Q6_K, *c) for c in few])) == {"D"}
+    rounds = [([6144], 512, 1100), ([14336], 512, 400), ([4096], 1024, 1024)]
+    assert "E" not in _prefill(route, [(TYPE_Q6_K, *c) for c in rounds])
+    many = [([2560], 9728, 512), ([4096], 4096, 512), ([4096], 512, 512), ([6144], 9728, 256)]
+    assert set(_prefill(route, [(TYPE_Q6_K, *c) for c in many])) == {"E"}
