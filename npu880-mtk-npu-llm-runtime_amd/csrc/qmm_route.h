@@ -119,4 +119,45 @@ inline Prefill prefill_kernel(KFormat f, const RowTiles &r, int K, int M, int cu
     return decoded ? Prefill::D128 : Prefill::P64x32;
 }
 
+// Up to 64 tokens: wave slabs of 64 rows and all the tokens, in 4 waves (their
+// 16-token tiles; 0: the small-M kernels). Those read every token's codes again
+// for each 16 rows (at 16-row tiles about 12 TB/s out of the L2s, their bound)
+// and again the rows for each token group; here 64 rows share them. Measured (K
+// = 2560 unless said, us, small-M kernel -> this): M = 48 at 19456 / 30000 /
+// 100000 rows Q4_K 23.4 / 32.6 / 98.7 -> 21.1 / 22.1 / 68.7, Q6_K 27.3 / 40.7 /
+// 121 -> 25.3 / 27.3 / 81.9, Q5_K 30000 x 4096 57.2 -> 36.3; M = 64 Q4_K 24.1 /
+// 34.0 / 102 -> 23.5 / 24.7 / 74.3.
+// Under one workgroup per CU (9728 rows at M = 37..64: 12.2..16 against
+// 15.3..19) a step's latency shows and the small-M kernels stay. So they do
+// where the last round of workgroups (one per CU each) is too empty, by how
+// good they are at that K: 33..64 tokens, time against theirs at 1.0 / 1.06 /
+// 1.19 / 1.25 / 1.38 / 2.02 workgroups per CU: K <= 1536 at most 0.94; K =
+// 2048..3072 (part kernel) 0.9 / 1.0..1.1 / 1.0 / 0.95 / 0.9 / 0.95; Q5_K and
+// Q6_K past that at most 0.97; Q4_K at K = 3584..4096 0.9 / 1.0 / 0.85 / 0.85 /
+// 0.8 / 0.85, past it 1.03 / 1.04 / 1.03 / 1.03 / 1.0 / 1.05 and 0.8 at 2.0.
+// Q4_K over K > 2560 at exactly one round 1.06.
+// At 17..32 tokens the small-M kernels take each 16-row tile's tokens at once:
+// faster here only for Q4_K from 7/4 workgroups per CU (30000 / 100000 rows
+// 20.6 / 55.2 -> 18.3 / 48.9). Time against theirs with the weights in HBM and
+// 2 GB of others read since, at 2.0 / 2.44 / 2.69 / 3.01 / 6.11 workgroups per
+// CU: K <= 1536 and K > 3072 at most 0.98, K = 2560 0.89 / 0.98 / 0.93 / 1.02 /
+// 0.94, K = 3072 (the part kernel's best) 0.95 / 1.03 / 0.97 / 1.10 / 1.05.
+// At 9..16 tokens Q6_K alone gains (decoding bound, one stage pair and four
+// waves per SIMD; K = 1024 / 1536 / 4096 on 151936 rows warm 0.71 / 0.80 / 0.83
+// of the part kernel's time, with the weights in HBM 0.73 / 0.85 / 0.83). Over
+// K = 2048..3072 it gains 0..10 % warm only: with the weights in HBM 1.0..1.05,
+// and 1.1..1.2 on buffers just written (a wave's 16 rows are 16 distant pieces
+// a step; the part kernel's are contiguous): left to the part kernel.
+inline int tall_tiles(KFormat f, int r64, int K, int M, int cus) {
+    if (M <= 8 || M > 64 || r64 < cus) return 0;
+    const int full = (r64 + cus - 1) / cus * cus;  // the rounds' slots
+    auto filled = [&](int num, int den) { return int64_t(den) * r64 > int64_t(num) * full; };
+    const bool q4 = f == KFormat::Q4;
+    if (M <= 16) return f == KFormat::Q6 && r64 >= 4 * cus && (K < 2048 || K > 3072) ? 1 : 0;
+    if (M <= 32) return q4 && 4 * r64 >= 7 * cus && (K <= 1536 || K > 3072 || (K <= 2560 && filled(4, 5))) ? 2 : 0;
+    const bool ok = K <= 1536 || (K <= 3072 || (q4 && K <= 4096) ? filled(5, 8) : !q4 || filled(3, 4));
+    if (!ok || (q4 && K > 2560 && r64 == cus)) return 0;
+    return (M + 15) / 16;
+}
+
 }  // namespace qmm

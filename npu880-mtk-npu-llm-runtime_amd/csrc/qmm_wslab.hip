@@ -283,35 +283,19 @@ hipError_t launch_wslab(Prefill p, const MatArgs *tasks, int n, const Q8KView &x
     return launch_wslab_t<WsCfg<F, 4, 4, 3>, F>(tasks, n, x, s);
 }
 
-// Up to 64 tokens: one group of all the tokens, 64 rows in 4 waves, three
-// stages (two blocks in flight: a block's work is short). The small-M kernels
-// read every token's codes again for each 16 rows (at 16-row tiles about 12
-// TB/s out of the L2s, their bound) and again the rows for each token group;
-// here 64 rows share them. Measured (K = 2560 unless said, us, small-M kernel
-// -> this): M = 48 at 19456 / 30000 / 100000 rows Q4_K 23.4 / 32.6 / 98.7 ->
-// 21.1 / 22.1 / 68.7, Q6_K 27.3 / 40.7 / 121 -> 25.3 / 27.3 / 81.9, Q5_K 30000
-// x 4096 57.2 -> 36.3; M = 64 Q4_K 24.1 / 34.0 / 102 -> 23.5 / 24.7 / 74.3.
-// Under one workgroup per CU (9728 rows at M = 37..64: 12.2..16 against
-// 15.3..19) a step's latency shows and the small-M kernels stay. At 17..32
-// tokens they take each 16-row tile's tokens at once: faster here only for
-// Q4_K from 7/4 workgroups per CU (30000 / 100000 rows 20.6 / 55.2 -> 18.3 /
-// 48.9). At 9..16 tokens Q6_K alone gains (decoding bound, one stage pair and
-// four waves per SIMD): 151936 rows 82 -> 79, 100000 x 4096 97 -> 86.
+// Up to 64 tokens (tall_tiles): one group of all the tokens, 64 rows in 4
+// waves, from 17 tokens three stages (two blocks in flight: a block's work is
+// short).
 template <class F>
 hipError_t launch_wslab_tall(const MatArgs *tasks, int n, const Q8KView &x, hipStream_t s) {
-    const int M = tasks[0].M, cus = mfma_cu_count();
-    int s64 = 0;
-    for (int i = 0; i < n; ++i) s64 += (tasks[i].N + 63) / 64;
-    if (M <= 8 || M > 64 || s64 < cus || !slab_ok<F>(tasks, n, x)) return hipErrorNotSupported;
-    // (Q5_K and Q6_K gain less: a few CUs with a second workgroup undo it, 16400
-    // rows at M = 60 25.9 against 27.0)
-    if (M > 32 && !std::is_same_v<F, MQ4KS> && s64 > cus && 8 * s64 < 9 * cus) return hipErrorNotSupported;
-    if (M > 48) return launch_wslab_t<WsCfg<F, 4, 4, 2, 3>, F>(tasks, n, x, s);
-    if (M > 32) return launch_wslab_t<WsCfg<F, 3, 4, 2, 3>, F>(tasks, n, x, s);
+    const int tt = tall_tiles(kformat<F>(), row_tiles(tasks, n).r64, tasks[0].K, tasks[0].M, mfma_cu_count());
+    if (!tt || !slab_ok<F>(tasks, n, x)) return hipErrorNotSupported;
+    if (tt == 4) return launch_wslab_t<WsCfg<F, 4, 4, 2, 3>, F>(tasks, n, x, s);
+    if (tt == 3) return launch_wslab_t<WsCfg<F, 3, 4, 2, 3>, F>(tasks, n, x, s);
     if constexpr (std::is_same_v<F, MQ4KS>)
-        if (M > 16 && 4 * s64 >= 7 * cus) return launch_wslab_t<WsCfg<F, 2, 4, 3, 3>, F>(tasks, n, x, s);
+        if (tt == 2) return launch_wslab_t<WsCfg<F, 2, 4, 3, 3>, F>(tasks, n, x, s);
     if constexpr (std::is_same_v<F, MQ6KS>)
-        if (M <= 16 && s64 >= 4 * cus) return launch_wslab_t<WsCfg<F, 1, 4, 4, 2>, F>(tasks, n, x, s);
+        if (tt == 1) return launch_wslab_t<WsCfg<F, 1, 4, 4, 2>, F>(tasks, n, x, s);
     return hipErrorNotSupported;
 }
 

@@ -49,6 +49,10 @@ int main() {
                 r.add(rows);
             }
             std::printf("%c\n", char(qmm::prefill_kernel(qmm::KFormat(f - 4), r, K, M, cus)));
+        } else if (!std::strcmp(what, "tall")) {  // format, rows, K, M, CUs: token tiles of the tall wave slabs
+            int f, rows, K, M, cus;
+            if (std::scanf("%d %d %d %d %d", &f, &rows, &K, &M, &cus) != 5) return 1;
+            std::printf("%d\n", qmm::tall_tiles(qmm::KFormat(f - 4), (rows + 63) / 64, K, M, cus));
         } else {
             return 1;
         }

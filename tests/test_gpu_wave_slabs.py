@@ -63,12 +63,15 @@ def test_decoded_slabs_256_tokens(ctx, oracle, type_id, rows, K, M, residual):
     _run(ctx, oracle, type_id, rows, K, M, residual)
 
 
-@pytest.mark.parametrize("type_id,rows,K,M,residual", [
-    # 64 rows x 64, 48, 32 and 16 tokens: one block (fewer than the stages), two, three and more; ragged tokens and rows
+# 64 rows x 64, 48, 32 and 16 tokens: one block (fewer than the stages), two, three and more; ragged tokens and rows
+TALL = [
     (TYPE_Q4_K, [16400], 256, 64, True), (TYPE_Q5_K, [20001], 512, 50, False), (TYPE_Q6_K, [19000], 768, 49, False),
     (TYPE_Q4_K, [9728, 9700], 1280, 37, True), (TYPE_Q5_K, [19456], 256, 48, False), (TYPE_Q6_K, [20003], 512, 33, True),
     (TYPE_Q4_K, [30000], 768, 17, False), (TYPE_Q4_K, [29001], 256, 32, True),
-    (TYPE_Q6_K, [65600], 256, 9, True), (TYPE_Q6_K, [65537], 768, 16, False)])
+    (TYPE_Q6_K, [65600], 256, 9, True), (TYPE_Q6_K, [65537], 768, 16, False)]
+
+
+@pytest.mark.parametrize("type_id,rows,K,M,residual", TALL)
 def test_wave_slabs_tall(ctx, oracle, type_id, rows, K, M, residual):
     _run(ctx, oracle, type_id, rows, K, M, residual)
 

@@ -6,7 +6,7 @@ import subprocess
 import pytest
 
 from oracle import TYPE_Q4_K, TYPE_Q5_K, TYPE_Q6_K
-from test_gpu_wave_slabs import PREFILL
+from test_gpu_wave_slabs import PREFILL, TALL
 
 FORMAT = {TYPE_Q4_K: 4, TYPE_Q5_K: 5, TYPE_Q6_K: 6}
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -71,3 +71,28 @@ def test_prefill_q6k_256_tokens_only_where_faster(route):
     assert "E" not in _prefill(route, [(TYPE_Q6_K, *c) for c in rounds])
     many = [([2560], 9728, 512), ([4096], 4096, 512), ([4096], 512, 512), ([6144], 9728, 256)]
     assert set(_prefill(route, [(TYPE_Q6_K, *c) for c in many])) == {"E"}
+
+
+def _tall(route, cases):
+    return [int(v) for v in route([f"tall {FORMAT[t]} {rows} {K} {M} 256" for t, rows, K, M in cases])]
+
+
+def test_tall_kernels_of_the_gpu_cases(route):
+    cases = [(t, sum(64 * -(-n // 64) for n in rows), K, M) for t, rows, K, M, _ in TALL]
+    assert _tall(route, cases) == [(c[3] + 15) // 16 for c in cases]
+
+
+def test_tall_wave_slabs_only_where_faster(route):
+    """Not under one workgroup of 64 rows per CU, not where the last round is too
+    empty for the K, and at 32 tokens or fewer not at the K that the part kernel
+    reads best (all of these measured slower than the small-M kernels)."""
+    q4, q5, q6 = TYPE_Q4_K, TYPE_Q5_K, TYPE_Q6_K
+    slower = [(q4, 9728, 2560, 64), (q4, 18432, 2560, 49), (q5, 18432, 2560, 33), (q5, 19456, 2560, 33),
+              (q6, 18432, 2560, 64), (q4, 16384, 3072, 33), (q4, 33000, 9728, 33), (q4, 19456, 9728, 49),
+              (q4, 33000, 2560, 17), (q4, 38000, 3072, 32), (q4, 49300, 3072, 24), (q6, 66000, 3072, 12),
+              (q6, 151936, 2560, 16), (q6, 100000, 2048, 9)]
+    assert _tall(route, slower) == [0] * len(slower)
+    faster = [(q4, 28672, 2560, 64), (q5, 16384, 2560, 49), (q6, 18432, 4096, 49), (q5, 17408, 8192, 33),
+              (q4, 33000, 4096, 17), (q4, 44000, 2560, 24), (q6, 151936, 1024, 16), (q6, 100000, 4096, 9),
+              (q6, 18432, 1024, 33)]
+    assert _tall(route, faster) == [(c[3] + 15) // 16 for c in faster]
