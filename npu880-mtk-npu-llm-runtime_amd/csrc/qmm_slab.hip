@@ -1,17 +1,15 @@
 // qmm_slab.hip — prefill GEMM (M > 64 tokens) over GGUF-packed k-quant rows
 // (Q4_K, Q5_K, Q6_K) with int8 MFMA, gfx950.
 //
-// Workgroup = NW (4 or 8) waves on a slab of R = 16 RW PR weight rows x
-// T = 16 TW PT tokens; wave (pr, pt) owns RW row tiles x TW token tiles of
-// 16 x 16. The K
-// loop walks one 256-value block at a time through PD LDS stages, each filled by direct buffer -> LDS
-// transfers (buffer_load ... lds): the slab's packed weight rows, the
-// tokens' codes from the tiles section of the activation buffer (already in
+// Packed slabs (slab_kernel): a workgroup is 4 waves on 64 weight rows x 32
+// tokens; a wave owns 16 rows x both token tiles. The K loop walks one
+// 256-value block at a time through two LDS stages, each filled by direct
+// buffer -> LDS transfers (buffer_load ... lds): the slab's packed weight rows,
+// the tokens' codes from the tiles section of the activation buffer (already in
 // MFMA operand order), their fp16 sums of 16 codes (bh section) and their
-// block scales. A wave unpacks each of its row tiles once per step into
-// registers (the unit scales folded into two int8 B operands, as the small-M
-// kernels do) and reuses it for all TW token tiles, so the unpacking is paid
-// once per 16 TW tokens.
+// block scales. A wave unpacks its rows once per step into registers (the unit
+// scales folded into two int8 B operands, as the small-M kernels do) and uses
+// them for both token tiles. Decoded slabs (dslab_kernel): below.
 //
 // Per 16 x 16 tile and block: S = 8 D1 + D2 (Q4_K) or 256 D1 + D2 (Q5_K,
 // Q6_K) from two v_mfma_i32_16x16x64_i8 chains over the block's four 64-value
@@ -31,15 +29,11 @@
 
 namespace qmm {
 
-template <class F, int RW_, int TW_, int PR_, int PD_, int NW_ = 4, int WPS_ = 1>
+template <class F>
 struct SlabCfg {
-    static constexpr int NW = NW_;    // waves per workgroup
-    static constexpr int WPS = WPS_;  // waves per SIMD the registers must allow (launch bound)
-    static constexpr int RW = RW_, TW = TW_, PR = PR_, PT = NW_ / PR_, PD = PD_;
-    static_assert(PR * PT == NW, "PR x PT waves");
+    static constexpr int NW = 4, TW = 2;  // waves, token tiles
     static constexpr bool MIN = F::kMin;
-    static constexpr int R = 16 * RW * PR;  // weight rows per workgroup
-    static constexpr int T = 16 * TW * PT;  // tokens per workgroup
+    static constexpr int R = 16 * NW, T = 16 * TW;  // weight rows, tokens per workgroup
     static constexpr int SB = F::BB;  // weight bytes per row and step
     // rows of Q4_K / Q5_K start 16-B aligned (the launcher checks):
     // a step's bytes are whole 16-B units; Q6_K's 210-B blocks take the 16-B
@@ -52,25 +46,22 @@ struct SlabCfg {
     static constexpr int NDI = (T + 63) / 64;                        // scales (4-B transfers)
     static constexpr int NWW = (NWI + NW - 1) / NW, NAW = NAI / NW, NBW = (NBI + NW - 1) / NW,
                          NDW = (NDI + NW - 1) / NW;
-    static constexpr int L = NWW + NAW + NBW + NDW;       // transfers per wave and step
     static constexpr int OFF_A = NWI * 1024;
     static constexpr int OFF_B = OFF_A + NAI * 1024;
     static constexpr int OFF_D = OFF_B + NBI * 1024;
     static constexpr int STAGE = OFF_D + NDI * 256;
-    static constexpr int OFF_DUMP = PD * STAGE, LDS = OFF_DUMP + 1024;
+    static constexpr int OFF_DUMP = 2 * STAGE, LDS = OFF_DUMP + 1024;
     static_assert(NAI % NW == 0, "code transfers: a multiple of the waves");
-    static_assert((PD - 2) * L <= 63, "vmcnt range");
     static_assert(LDS <= 160 * 1024, "LDS");
 };
 
 template <class C, class F>
-__global__ __launch_bounds__(64 * C::NW, C::WPS) void slab_kernel(MatGroup grp, typename ActOf<F>::T x, int ntg) {
+__global__ __launch_bounds__(64 * C::NW) void slab_kernel(MatGroup grp, typename ActOf<F>::T x, int ntg) {
     extern __shared__ __align__(16) uint8_t lds[];
-    constexpr int RW = C::RW, TW = C::TW;
+    constexpr int TW = C::TW;
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nl = lane & 15, cl = lane >> 4;
-    const int pt = wid % C::PT, pr = wid / C::PT;
 
     // workgroup -> (row slab, token group): consecutive slots of one XCD
     // take the token groups of one slab
@@ -130,7 +121,7 @@ __global__ __launch_bounds__(64 * C::NW, C::WPS) void slab_kernel(MatGroup grp, 
         dof[s] = p < C::T ? uint32_t(m0 + p) * uint32_t(nbk) * 4u : kFar;
     }
     const uint32_t wrange = uint32_t(rw.z), arange = uint32_t(ra.z), brange = uint32_t(rb.z), drange = uint32_t(rd.z);
-    // the transfers of step st into stage sg (every wave issues L per step)
+    // the transfers of step st into stage sg
     auto issue = [&](int st, int sg) __attribute__((always_inline)) {
         const bool live = st < nsteps;
         const uint32_t base = lds0 + uint32_t(sg * C::STAGE), dump = lds0 + uint32_t(C::OFF_DUMP);
@@ -161,32 +152,26 @@ __global__ __launch_bounds__(64 * C::NW, C::WPS) void slab_kernel(MatGroup grp, 
         }
     };
 
-    float acc[RW][TW][4];
+    float acc[TW][4];
 #pragma unroll
-    for (int r = 0; r < RW; ++r)
+    for (int t = 0; t < TW; ++t)
 #pragma unroll
-        for (int t = 0; t < TW; ++t)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) acc[r][t][q] = 0.0f;
+        for (int q = 0; q < 4; ++q) acc[t][q] = 0.0f;
 
-#pragma unroll
-    for (int p = 0; p + 1 < C::PD; ++p) issue(p, p);
+    issue(0, 0);
     for (int st = 0; st < nsteps; ++st) {
-        const int sg = st % C::PD;
-        wait_vmcnt<(C::PD - 2) * C::L>();  // this wave's transfers of step st have landed
-        __builtin_amdgcn_s_barrier();       // every wave's have; stage (st - 1) is free
+        const int sg = st % 2;
+        wait_vmcnt<0>();               // this wave's transfers of step st have landed
+        __builtin_amdgcn_s_barrier();  // every wave's have; the other stage is free
         __builtin_amdgcn_sched_barrier(0);
-        issue(st + C::PD - 1, (st + C::PD - 1) % C::PD);
+        issue(st + 1, (st + 1) % 2);
         const uint8_t *sbase = lds + sg * C::STAGE;
         const uint8_t *sa = sbase + C::OFF_A;
         const float *sd = reinterpret_cast<const float *>(sbase + C::OFF_D);
-        SlabB B[RW];
-#pragma unroll
-        for (int r = 0; r < RW; ++r) {
-            const int rl = (pr * RW + r) * 16 + nl;  // lane's row in the slab
-            const uint32_t mis = C::ALIGNED ? 0u : (uint32_t(rl) * uint32_t(a.row_bytes) + bl + uint32_t(st) * uint32_t(C::SB)) & 15u;
-            slab_unpack<F>(sbase + rl * (C::WCR * 16) + mis, cl, B[r]);
-        }
+        SlabB B;
+        const int rl = wid * 16 + nl;  // lane's row in the slab
+        const uint32_t mis = C::ALIGNED ? 0u : (uint32_t(rl) * uint32_t(a.row_bytes) + bl + uint32_t(st) * uint32_t(C::SB)) & 15u;
+        slab_unpack<F>(sbase + rl * (C::WCR * 16) + mis, cl, B);
         {
             // tile u: codes and sums loaded two tiles ahead, dx one ahead; the
             // MFMAs of tile t + 1 are issued before tile t's fp32 update, so
@@ -194,49 +179,43 @@ __global__ __launch_bounds__(64 * C::NW, C::WPS) void slab_kernel(MatGroup grp, 
             uint4 av[2][4];
             half4v bh[2];
             float4 dx[2];
-            int4v D1[2][RW], D2[2][RW];
-            f32x4v Mb[2][RW];
+            int4v D1[2], D2[2];
+            f32x4v Mb[2];
             auto load_a = [&](int t, int buf) __attribute__((always_inline)) {
-                const int tt = pt * TW + t;
 #pragma unroll
-                for (int h = 0; h < 4; ++h) av[buf][h] = ld16(sa + (tt * 4 + h) * 1024 + 16 * lane);
-                if constexpr (C::MIN) bh[buf] = __builtin_bit_cast(half4v, ld8(sbase + C::OFF_B + tt * 512 + 8 * lane));
+                for (int h = 0; h < 4; ++h) av[buf][h] = ld16(sa + (t * 4 + h) * 1024 + 16 * lane);
+                if constexpr (C::MIN) bh[buf] = __builtin_bit_cast(half4v, ld8(sbase + C::OFF_B + t * 512 + 8 * lane));
             };
             auto load_d = [&](int t, int buf) __attribute__((always_inline)) {
-                dx[buf] = *reinterpret_cast<const float4 *>(sd + (pt * TW + t) * 16 + 4 * cl);
+                dx[buf] = *reinterpret_cast<const float4 *>(sd + t * 16 + 4 * cl);
             };
             auto mm = [&](int buf) __attribute__((always_inline)) {
+                int4v d1 = {0, 0, 0, 0}, d2 = {0, 0, 0, 0};
 #pragma unroll
-                for (int r = 0; r < RW; ++r) {
-                    int4v d1 = {0, 0, 0, 0}, d2 = {0, 0, 0, 0};
-#pragma unroll
-                    for (int h = 0; h < 4; ++h) {
-                        d1 = mfma16x16x64(av[buf][h], B[r].b1[h], d1);
-                        d2 = mfma16x16x64(av[buf][h], B[r].b2[h], d2);
-                    }
-                    D1[buf][r] = d1;
-                    D2[buf][r] = d2;
-                    f32x4v m = {0.0f, 0.0f, 0.0f, 0.0f};
-                    if constexpr (C::MIN) m = __builtin_amdgcn_mfma_f32_16x16x16f16(bh[buf], B[r].mh, m, 0, 0, 0);
-                    Mb[buf][r] = m;
+                for (int h = 0; h < 4; ++h) {
+                    d1 = mfma16x16x64(av[buf][h], B.b1[h], d1);
+                    d2 = mfma16x16x64(av[buf][h], B.b2[h], d2);
                 }
+                D1[buf] = d1;
+                D2[buf] = d2;
+                f32x4v m = {0.0f, 0.0f, 0.0f, 0.0f};
+                if constexpr (C::MIN) m = __builtin_amdgcn_mfma_f32_16x16x16f16(bh[buf], B.mh, m, 0, 0, 0);
+                Mb[buf] = m;
             };
             auto epi = [&](int t, int buf) __attribute__((always_inline)) {
                 const float dxq[4] = {dx[buf].x, dx[buf].y, dx[buf].z, dx[buf].w};
 #pragma unroll
-                for (int r = 0; r < RW; ++r)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const int S = (D1[buf][r][q] << F::kShift) + D2[buf][r][q];
-                        if constexpr (C::MIN)
-                            acc[r][t][q] += dxq[q] * (B[r].d * (float)S - B[r].dmin * Mb[buf][r][q]);  // E:11026 / E:11063
-                        else
-                            acc[r][t][q] += (B[r].d * dxq[q]) * (float)S;  // E:11101
-                    }
+                for (int q = 0; q < 4; ++q) {
+                    const int S = (D1[buf][q] << F::kShift) + D2[buf][q];
+                    if constexpr (C::MIN)
+                        acc[t][q] += dxq[q] * (B.d * (float)S - B.dmin * Mb[buf][q]);  // E:11026 / E:11063
+                    else
+                        acc[t][q] += (B.d * dxq[q]) * (float)S;  // E:11101
+                }
             };
             load_a(0, 0);
             load_d(0, 0);
-            if (TW > 1) load_a(1, 1);
+            load_a(1, 1);
             mm(0);
 #pragma unroll
             for (int t = 0; t < TW; ++t) {
@@ -248,7 +227,7 @@ __global__ __launch_bounds__(64 * C::NW, C::WPS) void slab_kernel(MatGroup grp, 
                 epi(t, t & 1);
                 if (t + 1 < TW) {
 #pragma unroll
-                    for (int i = 0; i < (C::MIN ? 9 : 8) * RW; ++i) {
+                    for (int i = 0; i < (C::MIN ? 9 : 8); ++i) {
                         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA of tile t + 1
                         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read of tile t + 2
                         __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);  // three VALU of tile t's update
@@ -259,21 +238,18 @@ __global__ __launch_bounds__(64 * C::NW, C::WPS) void slab_kernel(MatGroup grp, 
     }
     wait_vmcnt<0>();  // the tail's transfers (zeros into a free stage) land before the workgroup ends
 
+    const int n = n0 + wid * 16 + nl;
+    if (n >= a.N) return;
 #pragma unroll
-    for (int r = 0; r < RW; ++r) {
-        const int n = n0 + (pr * RW + r) * 16 + nl;
-        if (n >= a.N) continue;
+    for (int t = 0; t < TW; ++t)
 #pragma unroll
-        for (int t = 0; t < TW; ++t)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int tok = m0 + (pt * TW + t) * 16 + 4 * cl + q;
-                if (tok >= a.M) continue;
-                float v = acc[r][t][q];
-                if (a.res) v = v + a.res[size_t(tok) * a.ldr + n];
-                a.y[size_t(tok) * a.ldy + n] = v;
-            }
-    }
+        for (int q = 0; q < 4; ++q) {
+            const int tok = m0 + t * 16 + 4 * cl + q;
+            if (tok >= a.M) continue;
+            float v = acc[t][q];
+            if (a.res) v = v + a.res[size_t(tok) * a.ldr + n];
+            a.y[size_t(tok) * a.ldy + n] = v;
+        }
 }
 
 // ------------------------------------------------------------ decoded slabs
@@ -854,7 +830,7 @@ hipError_t launch_slab(const MatArgs *tasks, int n, const typename ActOf<F>::T &
     // 64 rows x 32 tokens in 4 waves, three or four workgroups per CU (O 2560
     // x 4096 at M = 512: 28.5 -> 23.9 us against 64 x 64). Measured slower at
     // M = 512: 32 x 64, 64 x 16, 32 x 32, three stages, two row tiles per wave.
-    return launch_slab_t<SlabCfg<F, 1, 2, 4, 2>, F>(tasks, n, x, s);
+    return launch_slab_t<SlabCfg<F>, F>(tasks, n, x, s);
 }
 
 template hipError_t launch_slab<MQ4KS>(const MatArgs *, int, const Q8KView &, hipStream_t);
