@@ -276,9 +276,10 @@ def _extreme_weights(type_id, N, K, seed):
 @pytest.mark.parametrize("type_id", [TYPE_Q4_K, TYPE_Q5_K, TYPE_Q6_K])
 @pytest.mark.parametrize("M,K", [(5, 1024), (40, 1024), (512, 1024), (512, 4352), (40, 4352)])
 def test_mfma_extreme_scales(ctx, oracle, type_id, M, K):
-    """Extreme scales and quants through the MFMA paths (scales folded into
-    the weight operand from M > 16; the slab kernels over K > 4096): the
-    integer sums stay exact."""
+    """Extreme scales and quants through the MFMA paths of a short tensor
+    (scales folded into the weight operand from M > 16; the packed and decoded
+    slabs over K > 4096; tall tensors: test_gpu_wave_slabs.py): the integer
+    sums stay exact."""
     N = 96
     say(f"extreme scales {NAMES[type_id]} N={N} K={K} M={M}")
     w = _extreme_weights(type_id, N, K, seed=700 + M)
@@ -518,8 +519,8 @@ def test_task_groups_one_launch(ctx, oracle, M):
 
 @pytest.mark.parametrize("M,K,specs,residual", [(512, 2560, (9728, 9728), False), (300, 512, (13200, 13107), True)])
 def test_prefill_eight_wave_slabs(ctx, oracle, M, K, specs, residual):
-    """Task groups with at least four 128 x 64 slabs per CU take the 8-wave
-    prefill workgroups: the FFN's gate + up at M = 512, and ragged tasks
+    """Tall Q4_K task groups take the wave slabs of 128 rows x 64 tokens in 8
+    waves (test_route.py): the FFN's gate + up at M = 512, and ragged tasks
     (partial row slabs and token groups, a residual) at M = 300; one row of
     every 16-row tile of each task against the oracle, all tokens."""
     say(f"prefill 8-wave slabs M={M} K={K} tasks={specs}")
@@ -558,10 +559,10 @@ def test_prefill_eight_wave_slabs(ctx, oracle, M, K, specs, residual):
     (TYPE_Q6_K, 129, 4352, (2560,), None),
 ])
 def test_prefill_decoded_slab_groups(ctx, oracle, type_id, M, K, specs, res_task):
-    """Q5_K / Q6_K from 128 tokens take the decoded-slab workgroups: task
-    groups over their concatenated row slabs (partial slabs at each task's
-    end), partial token groups, a residual; every row of every task, all
-    tokens, against the oracle."""
+    """Q5_K / Q6_K calls that take the decoded slabs of 128 tokens (32 and 16
+    rows; test_route.py): task groups over their concatenated row slabs
+    (partial slabs at each task's end), partial token groups, a residual;
+    every row of every task, all tokens, against the oracle."""
     say(f"prefill decoded slabs {NAMES[type_id]} M={M} K={K} tasks={specs}")
     x = synth.activations(M, K, seed=3600 + M)
     xb = ctx.upload(x)

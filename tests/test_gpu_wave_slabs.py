@@ -1,7 +1,8 @@
-"""The wave-slab prefill GEMM (csrc/qmm_wslab.hip) vs the oracle, bit for bit:
-its three shapes (128 rows x 96 tokens, 128 x 64, 64 x 64) on every k-quant
-format, with rows and tokens past the last tile, one block and several, a
-task group, a residual, and Q6_K rows off every 16-B boundary."""
+"""The wave-slab GEMM (csrc/qmm_wslab.hip) vs the oracle, bit for bit: its
+prefill shapes (128 rows x 96 tokens, 128 x 64, 64 x 64) and its tall ones (up
+to 64 tokens) on every k-quant format, with rows and tokens past the last tile,
+one block and several, a task group, a residual, extreme scales, and Q6_K rows
+off every 16-B boundary."""
 import numpy as np
 import pytest
 
@@ -9,6 +10,7 @@ import qmm_hip
 import synth
 from gpu_util import check_outputs, say
 from oracle import TYPE_Q4_K, TYPE_Q5_K, TYPE_Q6_K
+from test_gpu_matmul import _extreme_weights as extreme_weights
 
 pytestmark = pytest.mark.gpu
 
@@ -74,6 +76,24 @@ TALL = [
 @pytest.mark.parametrize("type_id,rows,K,M,residual", TALL)
 def test_wave_slabs_tall(ctx, oracle, type_id, rows, K, M, residual):
     _run(ctx, oracle, type_id, rows, K, M, residual)
+
+
+# taller than the small-M and the other prefill kernels: tall slabs, and 128 x 96 / 64 x 64
+EXTREME = [(TYPE_Q4_K, 16400, 512, 40), (TYPE_Q5_K, 16400, 512, 40), (TYPE_Q6_K, 16400, 512, 40),
+           (TYPE_Q4_K, 3000, 512, 2000), (TYPE_Q5_K, 8201, 512, 300), (TYPE_Q6_K, 9001, 768, 300)]
+
+
+@pytest.mark.parametrize("type_id,rows,K,M", EXTREME)
+def test_wave_slabs_extreme_scales(ctx, oracle, type_id, rows, K, M):
+    """The largest scales, mins and quants: the integer sums stay exact."""
+    say(f"extreme scales type {type_id} rows={rows} K={K} M={M}")
+    w = extreme_weights(type_id, rows, K, seed=rows + M)
+    x = synth.activations(M, K, seed=701)
+    x[:, ::7] *= 50.0   # large entries: many codes at +-127
+    wb = ctx.weight_upload(w, type_id, rows, K)
+    y = ctx.gemm(type_id, wb, rows, K, x)
+    ctx.free(wb)
+    check_outputs(y, oracle.gemm_multi(x, [dict(w=w, type=type_id, rows=rows)])[0], f"extreme {type_id} M={M}")
 
 
 @pytest.mark.parametrize("rows,K,M", [([20000], 768, 40), ([66000], 768, 12), ([5000], 768, 1000), ([6000], 256, 600), ([9000], 768, 300)])

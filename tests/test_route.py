@@ -6,7 +6,7 @@ import subprocess
 import pytest
 
 from oracle import TYPE_Q4_K, TYPE_Q5_K, TYPE_Q6_K
-from test_gpu_wave_slabs import PREFILL, TALL
+from test_gpu_wave_slabs import EXTREME, PREFILL, TALL
 
 FORMAT = {TYPE_Q4_K: 4, TYPE_Q5_K: 5, TYPE_Q6_K: 6}
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -58,6 +58,18 @@ def test_prefill_kernels_of_the_gpu_cases(route):
     """Each case of the wave-slab GPU tests takes the kernel it is there for."""
     for kernel, cases in PREFILL.items():
         assert _prefill(route, [c[:4] for c in cases]) == [kernel] * len(cases), kernel
+    assert _prefill(route, [(t, [n], K, M) for t, n, K, M in EXTREME if M > 64]) == ["A", "C", "C"]
+    assert _tall(route, [c for c in EXTREME if c[3] <= 64]) == [3, 3, 3]
+
+
+def test_prefill_kernels_of_the_matmul_tests(route):
+    """test_gpu_matmul.py's tests of the 8-wave and the decoded slabs, and its
+    512-token layer (gate alone too)."""
+    q4, q5, q6 = TYPE_Q4_K, TYPE_Q5_K, TYPE_Q6_K
+    assert _prefill(route, [(q4, [9728, 9728], 2560, 512), (q4, [13200, 13107], 512, 300)]) == ["B", "B"]
+    assert _prefill(route, [(q5, [2048, 512, 528], 2560, 256), (q5, [4000, 1037], 1024, 333), (q6, [3000, 450], 1024, 384),
+                            (q6, [2560], 4352, 129), (q5, [9000], 2560, 65), (q5, [9000], 2560, 100)]) == ["D"] * 6
+    assert _prefill(route, [(q5, [6144], 2560, 512), (q4, [2560], 4096, 512), (q6, [2560], 9728, 512)]) == ["C", "P", "E"]
 
 
 def test_prefill_q6k_256_tokens_only_where_faster(route):
