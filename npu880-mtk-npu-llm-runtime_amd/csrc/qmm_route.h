@@ -132,10 +132,11 @@ inline Prefill prefill_kernel(KFormat f, const RowTiles &r, int K, int M, int cu
 // where the last round of workgroups (one per CU each) is too empty, by how
 // good they are at that K: 33..64 tokens, time against theirs at 1.0 / 1.06 /
 // 1.19 / 1.25 / 1.38 / 2.02 workgroups per CU: K <= 1536 at most 0.94; K =
-// 2048..3072 (part kernel) 0.9 / 1.0..1.1 / 1.0 / 0.95 / 0.9 / 0.95; Q5_K and
-// Q6_K past that at most 0.97; Q4_K at K = 3584..4096 0.9 / 1.0 / 0.85 / 0.85 /
-// 0.8 / 0.85, past it 1.03 / 1.04 / 1.03 / 1.03 / 1.0 / 1.05 and 0.8 at 2.0.
-// Q4_K over K > 2560 at exactly one round 1.06.
+// 2560 0.9 / 1.05 / 0.95 / 0.95 / 0.9 / 0.95, Q5_K at 33 tokens 1.0 / 1.1 /
+// 1.03 / 0.99 / 0.9 / 1.0; K = 3072 (the part kernel's best) 0.95 / 1.1 / 1.02 /
+// 1.0 / 0.9 / 0.97; Q5_K and Q6_K past that at most 0.97; Q4_K at K = 3584..4096
+// 0.9 / 1.0 / 0.85 / 0.85 / 0.8 / 0.85, past it 1.03 / 1.04 / 1.03 / 1.03 / 1.0 /
+// 1.05 and 0.8 at 2.0. Q4_K over K > 2560 at exactly one round 1.06.
 // At 17..32 tokens the small-M kernels take each 16-row tile's tokens at once:
 // faster here only for Q4_K from 7/4 workgroups per CU (30000 / 100000 rows
 // 20.6 / 55.2 -> 18.3 / 48.9). Time against theirs with the weights in HBM and
@@ -155,7 +156,10 @@ inline int tall_tiles(KFormat f, int r64, int K, int M, int cus) {
     const bool q4 = f == KFormat::Q4;
     if (M <= 16) return f == KFormat::Q6 && r64 >= 4 * cus && (K < 2048 || K > 3072) ? 1 : 0;
     if (M <= 32) return q4 && 4 * r64 >= 7 * cus && (K <= 1536 || K > 3072 || (K <= 2560 && filled(4, 5))) ? 2 : 0;
-    const bool ok = K <= 1536 || (K <= 3072 || (q4 && K <= 4096) ? filled(5, 8) : !q4 || filled(3, 4));
+    const bool ok = K <= 1536                         ? true
+                    : K <= 2560 && f != KFormat::Q5   ? filled(7, 12)
+                    : K <= 3072 || (q4 && K <= 4096) ? filled(5, 8)
+                                                      : !q4 || filled(3, 4);
     if (!ok || (q4 && K > 2560 && r64 == cus)) return 0;
     return (M + 15) / 16;
 }

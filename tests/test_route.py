@@ -100,11 +100,12 @@ def test_tall_wave_slabs_only_where_faster(route):
     reads best (all of these measured slower than the small-M kernels)."""
     q4, q5, q6 = TYPE_Q4_K, TYPE_Q5_K, TYPE_Q6_K
     slower = [(q4, 9728, 2560, 64), (q4, 18432, 2560, 49), (q5, 18432, 2560, 33), (q5, 19456, 2560, 33),
-              (q6, 18432, 2560, 64), (q4, 16384, 3072, 33), (q4, 33000, 9728, 33), (q4, 19456, 9728, 49),
+              (q6, 18432, 2560, 64), (q6, 19456, 3072, 64), (q4, 16384, 3072, 33), (q4, 33000, 9728, 33), (q4, 19456, 9728, 49),
               (q4, 33000, 2560, 17), (q4, 38000, 3072, 32), (q4, 49300, 3072, 24), (q6, 66000, 3072, 12),
               (q6, 151936, 2560, 16), (q6, 100000, 2048, 9)]
     assert _tall(route, slower) == [0] * len(slower)
-    faster = [(q4, 28672, 2560, 64), (q5, 16384, 2560, 49), (q6, 18432, 4096, 49), (q5, 17408, 8192, 33),
+    faster = [(q4, 28672, 2560, 64), (q4, 19456, 2560, 37), (q6, 19456, 2560, 48), (q5, 16384, 2560, 49),
+              (q6, 18432, 4096, 49), (q5, 17408, 8192, 33),
               (q4, 33000, 4096, 17), (q4, 44000, 2560, 24), (q6, 151936, 1024, 16), (q6, 100000, 4096, 9),
               (q6, 18432, 1024, 33)]
     assert _tall(route, faster) == [(c[3] + 15) // 16 for c in faster]
