@@ -941,6 +941,10 @@ PMC_WORKLOADS = [
     ("prefill_gate", synth.TYPE_Q4_K, 9728, 2560, 512),
     ("prefill_down", synth.TYPE_Q6_K, 2560, 9728, 512),
     ("prefill_q8_0", synth.TYPE_Q8_0, 2560, 2560, 512),
+    ("tree_gate_up_m37", synth.TYPE_Q4_K, 19456, 2560, 37),
+    ("lm_head_m16", synth.TYPE_Q6_K, 151936, 2560, 16),
+    ("prompt_gate_up", synth.TYPE_Q4_K, 19456, 2560, 2048),
+    ("prompt_down", synth.TYPE_Q6_K, 2560, 9728, 2048),
 ]
 PMC_MARKER_BASE = 1000  # workgroups of the marker launch before workload i: 1000 + i
 
@@ -1021,7 +1025,8 @@ def pmc_write(dirs):
     print("#     SQ_VALU_MFMA_COEXEC_CYCLES SQ_BUSY_CYCLES SQ_INSTS_VALU_MFMA_MOPS_F16 -d prof/gpmc4 ...")
     print(f"# summary: {cmd}")
     print("# derived: mfma_busy_frac = SQ_VALU_MFMA_BUSY_CYCLES / (GRBM_GUI_ACTIVE / 8 XCDs * 1024 SIMDs)")
-    print("#   (rocprof's MfmaUtil); valu_per_mfma = SQ_INSTS_VALU / SQ_INSTS_MFMA; int8_ops_executed =")
+    print("#   (rocprof's MfmaUtil); valu_slot_frac = SQ_INSTS_VALU * 4 / the same SIMD cycles;")
+    print("#   valu_per_mfma = SQ_INSTS_VALU / SQ_INSTS_MFMA; int8_ops_executed =")
     print("#   SQ_INSTS_VALU_MFMA_MOPS_I8 * 512; lds_bank_conflict_frac = SQ_LDS_BANK_CONFLICT / SQ_LDS_IDX_ACTIVE;")
     print("#   hbm_bytes = FETCH_SIZE * 1.9966 + WRITE_SIZE * 1.0 KiB (the factors the same counters read on a")
     print("#   device copy of known size, profiles/gemv_q4k_fused_9728x2560_pmc.txt); wave time (SQ_WAVE_CYCLES,")
@@ -1051,7 +1056,9 @@ def pmc_write(dirs):
             if c["SQ_INSTS_MFMA"] > 0:
                 print(f"{name}.valu_per_mfma: {c['SQ_INSTS_VALU'] / c['SQ_INSTS_MFMA']:.3f}")
         if "SQ_VALU_MFMA_BUSY_CYCLES" in c and c.get("GRBM_GUI_ACTIVE"):
-            print(f"{name}.mfma_busy_frac: {c['SQ_VALU_MFMA_BUSY_CYCLES'] / (c['GRBM_GUI_ACTIVE'] / 8 * 1024):.4f}")
+            simd = c["GRBM_GUI_ACTIVE"] / 8 * 1024
+            print(f"{name}.mfma_busy_frac: {c['SQ_VALU_MFMA_BUSY_CYCLES'] / simd:.4f}")
+            print(f"{name}.valu_slot_frac: {c['SQ_INSTS_VALU'] * 4 / simd:.4f}")
         if c.get("SQ_WAVE_CYCLES"):
             wc = c["SQ_WAVE_CYCLES"]
             for k, lab in (("SQ_ACTIVE_INST_VALU", "valu_active_frac"), ("SQ_WAIT_ANY", "wait_any_frac"),

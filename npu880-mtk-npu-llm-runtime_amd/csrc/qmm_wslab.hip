@@ -10,18 +10,22 @@
 // (two stages, shared by the NW waves); each wave's packed rows go through an
 // LDS region of its own with one stage only — free again as soon as the wave
 // has decoded it — which is what lets 96 tokens fit two workgroups of 8 waves
-// on a CU (74..81 KB of LDS, <= 128 VGPRs: four waves per SIMD).
+// on a CU (74..81 KB of LDS, <= 128 VGPRs: four waves per SIMD). At 96 tokens
+// that bound costs 3 spilled registers in Q4_K and 5 in Q5_K (none elsewhere):
+// transfer offsets reloaded from scratch inside the K loop, where the wait for
+// a reload is one for the transfers issued before it too.
 //
 // What bounds it: VALU issue, then power. A 16 x 16 tile and block costs 8
 // int8 MFMAs (128 cycles), 28 VALU of exact fp32 update (Q6_K: 20) and its
 // share of the decoding (Q4_K 94, Q5_K ~170, Q6_K 230 VALU per 16 rows and
-// block): at 96 tokens 69 % of all VALU issue slots are busy, the matrix core
-// 38 %, and the clock sits at 1.8 GHz. Shapes that trade these against each
+// block): Q4_K 19456 x 2560 at M = 2048 has 68 % of all VALU issue slots busy,
+// the matrix core 42 %, and the clock at 1.8 GHz (Q6_K 2560 x 9728 59 and 26 %;
+// at M = 512 33..50 % and 20 %). Shapes that trade these against each
 // other (32 x 32 MFMA tiles in two waves per SIMD, 192 tokens, no operand
 // reads at all) all land within 5 % of it. Measured (prequantized input,
 // kernel alone): down Q6_K 2560 x 9728 at M = 2048 230 -> 155 us, gate + up
-// Q4_K 2 x 9728 x 2560 at M = 2048 / 512 287 / 77 -> 264 / 70, QKV Q5_K 6144 x
-// 2560 at M = 2048 / 512 120 / 33.7 -> 102 / 29.9.
+// Q4_K 2 x 9728 x 2560 at M = 2048 / 512 287 / 77 -> 264 / 67, QKV Q5_K 6144 x
+// 2560 at M = 2048 / 512 120 / 33.7 -> 102 / 29.0.
 //
 // Arithmetic and results are the slab kernel's (qmm_slab.hip): exact integer
 // sums per block, the reference's fp32 expression, blocks in order.
