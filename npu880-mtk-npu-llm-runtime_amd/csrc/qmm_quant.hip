@@ -317,7 +317,8 @@ hipError_t launch_rmsnorm_q8k(const float *x, const float *gamma, int M, int K, 
     const unsigned grid = per ? unsigned(8 * per) : unsigned(M);
 #define QMM_RMS(NJ) \
     hipLaunchKernelGGL(rmsnorm_q8k_kernel<NJ>, dim3(grid), dim3(256), 0, s, x, gamma, M, K, per, y, o)
-    if (nj <= 3) QMM_RMS(3);
+    if (nj <= 1) QMM_RMS(1);
+    else if (nj <= 3) QMM_RMS(3);
     else if (nj <= 4) QMM_RMS(4);
     else if (nj <= 10) QMM_RMS(10);
     else if (nj <= 16) QMM_RMS(16);

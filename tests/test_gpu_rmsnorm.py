@@ -10,7 +10,7 @@ from gpu_util import check_q8k, say
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("M,K", [(1, 256), (1, 2560), (4, 4096), (3, 9728), (2, 16384), (3, 10240), (2, 10496)])
+@pytest.mark.parametrize("M,K", [(1, 256), (1, 2560), (4, 4096), (3, 9728), (2, 16384), (3, 10240), (2, 10496), (3, 1024)])
 def test_rmsnorm_q8k(ctx, oracle, M, K):
     say(f"rmsnorm_q8k M={M} K={K}")
     g = np.random.default_rng(M * 7 + K)
