@@ -20,22 +20,29 @@ constexpr int xcd_row(unsigned b, int per) { return per ? int(b % 8u) * per + in
 // of 9728 13.2 / 13.9 / 17.2 -> 12.4 / 13.2 / 16.5).
 constexpr int rms_rows_per_xcd(int M) { return M >= 256 ? (M + 7) / 8 : 0; }
 
-// The SwiGLU producer's workgroups take one token's quad of 256-value blocks.
-// A unit is one quad for 8 tokens, whose 16-B pieces of the tiles section fill
-// whole 128-B lines: 8 workgroups in a row on one XCD, which meet in its L2.
-// Units go round the XCDs, so no XCD takes more than one over another and the
-// launch walks memory in order. Measured (us; unit by unit / an eighth of the
-// 16-token tiles' quads to each XCD / blocks in order): 9728 columns at M = 17
-// / 65 / 513 / 2048 2.6 / 3.9 / 15.7 / 60.5, 3.0 / 4.4 / 15.2 / 61, 2.9 / 4.4
-// / 16.7 / 64.6; 9984 at M = 2048 61.6, 67.0, 64.3; 14336 88.9, 99.6, 98.8.
-struct QuadItem {
-    int m, q;  // token, quad
+// The SwiGLU producer: a wave takes one 256-value block of one token, wave by
+// wave an item (token, block). Per group of 8 tokens 2 nb workgroups of 4
+// waves, none without work: full quads of blocks first, each quad for the 8
+// tokens one after the other (their 16-B pieces of the tiles section fill whole
+// 128-B lines), then the last nb % 4 blocks, token by token. Of that sequence 8
+// workgroups in a row run on one XCD, and meet in its L2, the next 8 on the
+// next: no XCD takes more than 8 over another and the launch walks memory in
+// order. Measured (us; so / an eighth of the 16-token tiles' quads to each XCD,
+// a last quad's waves without a block idle / blocks in order): 9728 columns at M
+// = 17 / 65 / 513 / 2048 2.6 / 3.9 / 15.3 / 57.5, 3.0 / 4.4 / 15.2 / 61, 2.9 /
+// 4.4 / 16.8 / 65; 9984 at M = 2048 60.9, 67.0, 64.5; 14336 89.3, 99.6, 99.1;
+// 1280 at M = 2048 / 16384 8.9 / 62, 11.9 / 89, 9.8 / 72.
+struct BlockItem {
+    int m, j;  // token, block
 };
-constexpr QuadItem xcd_quad(unsigned b, int nq) {
-    const int i = int(b / 8u), u = (i >> 3) * 8 + int(b % 8u);
-    return QuadItem{u / nq * 8 + (i & 7), u % nq};
+constexpr BlockItem xcd_block(unsigned b, int wave, int nb) {
+    const int i = int(b / 8u), p = (i >> 3) * 64 + int(b % 8u) * 8 + (i & 7);
+    const int t = p / (2 * nb), w = p - t * 2 * nb, full = nb & ~3, r = nb & 3;
+    if (w < 2 * full) return BlockItem{8 * t + (w & 7), (w >> 3) * 4 + wave};
+    const int e = 4 * (w - 2 * full) + wave;  // (r > 0)
+    return BlockItem{8 * t + e / r, full + e % r};
 }
-constexpr unsigned xcd_quad_grid(int M, int nq) { return unsigned(((M + 7) / 8 * nq + 7) / 8 * 64); }
+constexpr unsigned xcd_block_grid(int M, int nb) { return (unsigned((M + 7) / 8) * unsigned(2 * nb) + 63u) / 64u * 64u; }
 
 enum class KFormat { Q4, Q5, Q6 };
 

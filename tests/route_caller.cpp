@@ -24,18 +24,19 @@ int main() {
             std::printf("%d", bad);
             for (int x : xcd) std::printf(" %d", x);
             std::printf("\n");
-        } else if (!std::strcmp(what, "quads")) {  // M, quads: items missed or taken twice, workgroups with work on each XCD
-            int M, nq;
-            if (std::scanf("%d %d", &M, &nq) != 2) return 1;
-            std::vector<int> seen(size_t(M) * nq), xcd(8);
+        } else if (!std::strcmp(what, "blocks")) {  // M, blocks: items missed or taken twice, waves with work on each XCD
+            int M, nb;
+            if (std::scanf("%d %d", &M, &nb) != 2) return 1;
+            std::vector<int> seen(size_t(M) * nb), xcd(8);
             int bad = 0;
-            for (unsigned b = 0; b < qmm::xcd_quad_grid(M, nq); ++b) {
-                const qmm::QuadItem it = qmm::xcd_quad(b, nq);
-                if (it.m >= M) continue;
-                if (it.q < 0 || it.q >= nq) return 1;
-                ++seen[size_t(it.m) * nq + it.q];
-                ++xcd[b % 8];
-            }
+            for (unsigned b = 0; b < qmm::xcd_block_grid(M, nb); ++b)
+                for (int wave = 0; wave < 4; ++wave) {
+                    const qmm::BlockItem it = qmm::xcd_block(b, wave, nb);
+                    if (it.m >= M) continue;
+                    if (it.j < 0 || it.j >= nb) return 1;
+                    ++seen[size_t(it.m) * nb + it.j];
+                    ++xcd[b % 8];
+                }
             for (int v : seen) bad += v != 1;
             std::printf("%d", bad);
             for (int x : xcd) std::printf(" %d", x);

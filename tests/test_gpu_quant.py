@@ -87,10 +87,10 @@ def test_swiglu_requant(ctx, oracle):
 
 
 @pytest.mark.parametrize("M,N", [(1, 1280), (7, 1024), (8, 256), (15, 2560), (16, 1024), (17, 2304), (37, 2048),
-                                 (300, 1280)])
-def test_swiglu_tokens_and_quads(ctx, oracle, M, N):
-    """Ragged units of 8 tokens and quads of blocks: every row and block written,
-    every section. The outputs start as bytes that no result has."""
+                                 (300, 1280), (9, 768), (20, 1792)])
+def test_swiglu_tokens_and_blocks(ctx, oracle, M, N):
+    """Ragged groups of 8 tokens and 0..3 blocks past the last quad: every row and
+    block written, every section. The outputs start as bytes that no result has."""
     say(f"swiglu tokens M={M} N={N}")
     g = synth.activations(M, N, seed=M + N) * 3
     u = synth.activations(M, N, seed=M + N + 1)

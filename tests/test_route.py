@@ -40,14 +40,16 @@ def test_rmsnorm_rows_cover_and_balance(route):
         assert max(xcd) <= (M + 7) // 8, (M, xcd)
 
 
-def test_swiglu_quads_cover_and_balance(route):
-    """Every token's every quad once; the XCDs' workgroups differ by at most one
-    unit of 8 tokens and one ragged unit."""
-    cases = [(M, nq) for M in (1, 7, 8, 9, 15, 16, 17, 37, 65, 100, 257, 300, 513, 2048) for nq in (1, 3, 10, 14)]
-    for (M, nq), line in zip(cases, route([f"quads {M} {nq}" for M, nq in cases])):
+def test_swiglu_blocks_cover_and_balance(route):
+    """Every token's every block once, no workgroup without a block but for
+    missing tokens; the XCDs' waves differ by at most two runs of 8 workgroups
+    (one run, and one of a ragged token group)."""
+    cases = [(M, nb) for M in (1, 7, 8, 9, 15, 16, 17, 37, 65, 100, 257, 300, 513, 2048)
+             for nb in (1, 2, 3, 4, 5, 6, 7, 9, 10, 38, 39, 56)]
+    for (M, nb), line in zip(cases, route([f"blocks {M} {nb}" for M, nb in cases])):
         bad, *xcd = map(int, line.split())
-        assert bad == 0 and sum(xcd) == M * nq, (M, nq, line)
-        assert max(xcd) - min(xcd) <= 8 + M % 8, (M, nq, xcd)
+        assert bad == 0 and sum(xcd) == M * nb, (M, nb, line)
+        assert max(xcd) - min(xcd) <= 64, (M, nb, xcd)
 
 
 def _prefill(route, cases):
