@@ -112,14 +112,14 @@ __global__ __launch_bounds__(256) void quantize_q8_0_kernel(const float *__restr
 
 // swiglu_chunk_worker (E:4349-4357): h = silu_mul(gate, up) per value, then
 // the fp16 round + Q8_K quantizer per 256-value block, a wave each. Bound by
-// memory (9728 columns at M = 2048: 57.5 us, 5.6 TB/s of the bytes it must
+// memory (9728 columns at M = 2048: 56.3 us, 5.7 TB/s of the bytes it must
 // move); waves placed by xcd_block.
 __global__ __launch_bounds__(256) void swiglu_q8k_kernel(const float *__restrict__ gate,
-                                                         const float *__restrict__ up, int M, int nb,
+                                                         const float *__restrict__ up, int M, BlockMap map,
                                                          float *__restrict__ h, Q8KOut o) {
-    const BlockItem it = xcd_block(blockIdx.x, int(threadIdx.x >> 6), nb);
-    const int m = it.m, j = it.j;
-    if (m >= M) return;
+    const BlockItem it = xcd_block(blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), map);
+    const int m = it.m, j = it.j, nb = map.nb;
+    if (m >= M || j >= nb) return;
     const size_t blk = size_t(m) * size_t(nb) + size_t(j);
     const int lane = threadIdx.x & 63;
     const float4 g = reinterpret_cast<const float4 *>(gate + blk * 256)[lane];
@@ -303,9 +303,8 @@ hipError_t launch_quantize_q8_0(const float *x, int M, int K, void *out, hipStre
 
 hipError_t launch_swiglu_q8k(const float *gate, const float *up, int M, int N, float *h,
                              void *out, hipStream_t s) {
-    const int nb = N / 256;
-    hipLaunchKernelGGL(swiglu_q8k_kernel, dim3(xcd_block_grid(M, nb)), dim3(256), 0, s, gate, up, M, nb, h,
-                       q8k_out(out, M, N));
+    const BlockMap map = block_map(M, N / 256);
+    hipLaunchKernelGGL(swiglu_q8k_kernel, dim3(map.grid), dim3(256), 0, s, gate, up, M, map, h, q8k_out(out, M, N));
     return hipGetLastError();
 }
 

@@ -20,29 +20,43 @@ constexpr int xcd_row(unsigned b, int per) { return per ? int(b % 8u) * per + in
 // of 9728 13.2 / 13.9 / 17.2 -> 12.4 / 13.2 / 16.5).
 constexpr int rms_rows_per_xcd(int M) { return M >= 256 ? (M + 7) / 8 : 0; }
 
-// The SwiGLU producer: a wave takes one 256-value block of one token, wave by
-// wave an item (token, block). Per group of 8 tokens 2 nb workgroups of 4
-// waves, none without work: full quads of blocks first, each quad for the 8
-// tokens one after the other (their 16-B pieces of the tiles section fill whole
-// 128-B lines), then the last nb % 4 blocks, token by token. Of that sequence 8
-// workgroups in a row run on one XCD, and meet in its L2, the next 8 on the
-// next: no XCD takes more than 8 over another and the launch walks memory in
+// The SwiGLU producer: a wave takes one 256-value block of one token, a
+// workgroup of 4 waves a quad of blocks, or one of the nb % 4 last blocks for 4
+// tokens, so that no wave is without a block. 8 workgroups in a row on one XCD
+// make a unit: a quad for a group of 8 tokens, or a last block for 32 tokens.
+// Their 16-B pieces of the tiles section fill whole 128-B lines in that XCD's
+// L2. Units go round the XCDs (none takes more than one over another), four
+// token groups' quads and then their last blocks: the launch walks memory in
 // order. Measured (us; so / an eighth of the 16-token tiles' quads to each XCD,
-// a last quad's waves without a block idle / blocks in order): 9728 columns at M
-// = 17 / 65 / 513 / 2048 2.6 / 3.9 / 15.3 / 57.5, 3.0 / 4.4 / 15.2 / 61, 2.9 /
-// 4.4 / 16.8 / 65; 9984 at M = 2048 60.9, 67.0, 64.5; 14336 89.3, 99.6, 99.1;
-// 1280 at M = 2048 / 16384 8.9 / 62, 11.9 / 89, 9.8 / 72.
-struct BlockItem {
-    int m, j;  // token, block
+// a last quad's waves without a block idle / blocks in order, every token's on
+// all XCDs): 9728 columns at M = 17 / 65 / 513 / 2048 2.6 / 3.85 / 14.6 / 56.3,
+// 3.0 / 4.4 / 15.2 / 61, 2.9 / 4.4 / 16.6 / 64.6; 9984 at M = 2048 59.8, 67.0,
+// 64.3; 14336 88.8, 99.6, 98.8; 1280 at M = 2048 / 16384 8.5 / 60, 11.9 / 89,
+// 9.8 / 72.
+struct BlockMap {
+    int nb, groups;  // blocks of a row, groups of 8 tokens
+    uint32_t inv;    // 2^32 / nb, rounded up: a unit's u inv / 2^32 is u / nb or one more
+    unsigned grid;   // workgroups
 };
-constexpr BlockItem xcd_block(unsigned b, int wave, int nb) {
-    const int i = int(b / 8u), p = (i >> 3) * 64 + int(b % 8u) * 8 + (i & 7);
-    const int t = p / (2 * nb), w = p - t * 2 * nb, full = nb & ~3, r = nb & 3;
-    if (w < 2 * full) return BlockItem{8 * t + (w & 7), (w >> 3) * 4 + wave};
-    const int e = 4 * (w - 2 * full) + wave;  // (r > 0)
-    return BlockItem{8 * t + e / r, full + e % r};
+constexpr BlockMap block_map(int M, int nb) {
+    const int groups = (M + 7) / 8, part = groups & 3;
+    const int units = (groups >> 2) * nb + (part ? part * (nb >> 2) + (nb & 3) : 0);
+    return BlockMap{nb, groups, uint32_t(0xFFFFFFFFu / unsigned(nb) + 1u), unsigned((units + 7) / 8) * 64u};
 }
-constexpr unsigned xcd_block_grid(int M, int nb) { return (unsigned((M + 7) / 8) * unsigned(2 * nb) + 63u) / 64u * 64u; }
+struct BlockItem {
+    int m, j;  // token, block (either may lie past the rows)
+};
+constexpr BlockItem xcd_block(unsigned b, int wave, const BlockMap &o) {
+    const int i = int(b / 8u), u = (i >> 3) * 8 + int(b % 8u), k = i & 7;
+    int s = o.nb > 1 ? int(uint64_t(unsigned(u)) * o.inv >> 32) : u, v = u - s * o.nb;
+    if (v < 0) --s, v += o.nb;
+    const int q = o.nb >> 2, left = o.groups - 4 * s, quads = (left < 4 ? left : 4) * q;
+    if (v < quads) {
+        const int g = int(v >= q) + int(v >= 2 * q) + int(v >= 3 * q);
+        return BlockItem{32 * s + 8 * g + k, 4 * (v - g * q) + wave};
+    }
+    return BlockItem{32 * s + 4 * k + wave, 4 * q + v - quads};
+}
 
 enum class KFormat { Q4, Q5, Q6 };
 

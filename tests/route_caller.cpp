@@ -29,11 +29,12 @@ int main() {
             if (std::scanf("%d %d", &M, &nb) != 2) return 1;
             std::vector<int> seen(size_t(M) * nb), xcd(8);
             int bad = 0;
-            for (unsigned b = 0; b < qmm::xcd_block_grid(M, nb); ++b)
+            const qmm::BlockMap map = qmm::block_map(M, nb);
+            for (unsigned b = 0; b < map.grid; ++b)
                 for (int wave = 0; wave < 4; ++wave) {
-                    const qmm::BlockItem it = qmm::xcd_block(b, wave, nb);
-                    if (it.m >= M) continue;
-                    if (it.j < 0 || it.j >= nb) return 1;
+                    const qmm::BlockItem it = qmm::xcd_block(b, wave, map);
+                    if (it.m < 0 || it.j < 0) return 1;
+                    if (it.m >= M || it.j >= nb) continue;
                     ++seen[size_t(it.m) * nb + it.j];
                     ++xcd[b % 8];
                 }

@@ -45,7 +45,7 @@ def test_swiglu_blocks_cover_and_balance(route):
     missing tokens; the XCDs' waves differ by at most two runs of 8 workgroups
     (one run, and one of a ragged token group)."""
     cases = [(M, nb) for M in (1, 7, 8, 9, 15, 16, 17, 37, 65, 100, 257, 300, 513, 2048)
-             for nb in (1, 2, 3, 4, 5, 6, 7, 9, 10, 38, 39, 56)]
+             for nb in (1, 2, 3, 4, 5, 6, 7, 9, 10, 38, 39, 56)] + [(12000, 4095)]  # (units past 2^32 / blocks)
     for (M, nb), line in zip(cases, route([f"blocks {M} {nb}" for M, nb in cases])):
         bad, *xcd = map(int, line.split())
         assert bad == 0 and sum(xcd) == M * nb, (M, nb, line)
